@@ -2,23 +2,27 @@
 //
 // quantize (fp8.py:28-49): per row, k = frexp(amax|x|).exponent - ebias and
 // q = fp8(x * 2^-k).  Three launch shapes:
-//   * rows that fit registers (<= 64 lanes x 16 vectors of 16 bytes: 8192
-//     bf16 / 4096 fp32 columns, 16-byte aligned): the row is read once into
-//     VGPRs, |x|max is a butterfly over the wave, and codes are written from
-//     the same registers: one HBM read and one write per element (3 B/elem
-//     for bf16 -> fp8).  Rows of up to 6 vectors per lane take one wave;
-//     longer ones are shared by a block's 4 waves, whose maxima meet in LDS,
-//     so that each wave holds at most 4 vectors and more rows stream at once.
-//     Each wave issues its loads one vector per lane at a time: fewer bytes
-//     in flight per CU keep the memory latency, and the bandwidth, up.
+//   * rows that fit registers (one vector up to 64 lanes x 16 vectors of 16
+//     bytes: 8 to 8192 bf16 / 4 to 4096 fp32 columns, any width and any
+//     element's alignment): the row is read once into VGPRs, |x|max is a
+//     butterfly over the wave, and codes are written from the same
+//     registers: one HBM read and one write per element (3 B/elem for bf16
+//     -> fp8).  Rows of up to 6 vectors per lane take one wave; longer ones
+//     are shared by a block's 4 waves, whose maxima meet in LDS, so that each
+//     wave holds at most 4 vectors and more rows stream at once.  A width
+//     that is no whole number of vectors ends in a vector that overlaps the
+//     one before it: [16376, 1601] bf16 quantizes in 17 us where element
+//     loads with two reads of x took 65 (79 MB: 4.5 against 1.2 TB/s).
+//     All of a row's loads are issued before the first is waited for (one
+//     vector at a time took C1's round trip from 30.0 to 32.0 us).
 //   * longer rows (per-tensor scaling is rows = 1): the row is cut into
 //     2048-element segments.  A first launch reduces the row's |x|max into
 //     at most 2,048 partial maxima (each wave strides over its row's
 //     segments; integer max, so order-free), a small second launch folds the
 //     partials per row, a third converts one segment per wave.  Two reads
 //     of x, no atomics.
-//   * any other shape (unaligned, columns not a multiple of the vector):
-//     the same two launches with element-wise loads.
+//   * any other shape (longer rows that are no whole aligned vectors, rows
+//     shorter than a vector): the same launches with element-wise loads.
 // Every row whose exponent keeps 2^-k, 2^k and every product exact
 // (|k| <= 110, finite |x|max) converts with the instructions: bf16 words go
 // straight into v_cvt_scalef32_pk_{fp8,bf8}_bf16 at scale 2^k (the code of
@@ -34,7 +38,9 @@
 // per lane per step for bf16 output (4 for fp32) so every store instruction
 // covers a contiguous 1 KB; bf16 output decodes with
 // v_cvt_scalef32_pk_bf16_{fp8,bf8} at scale 2^k unless the vector holds a
-// NaN code; roundtrip (fp8.py:56-63) fuses both.
+// NaN code; a vector that holds the end of one row and the start of the next
+// takes each code's own exponent ([16376, 1601] to bf16: 15 us, 41 code by
+// code); roundtrip (fp8.py:56-63) fuses both.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -64,9 +70,6 @@
 #ifndef ELY_SPLIT_BATCH
 #define ELY_SPLIT_BATCH 1  // split path: vectors per lane per load batch of the convert launch (0: all)
 #endif
-#ifndef ELY_Q_BATCH
-#define ELY_Q_BATCH 1  // register paths: vectors per lane per load batch (0: the whole row at once)
-#endif
 #ifndef ELY_Q_LDS
 // wave-per-row quantize: unused dynamic LDS per block, capping it at 16
 // blocks (16 waves) per CU.  C1 back to back over 8 inputs, in one process:
@@ -82,7 +85,7 @@
 #define ELY_RECOVER_KEEP_VPL 16  // longest rows (vectors per lane) whose image reuses the test's codes
 #endif
 #ifndef ELY_RECOVER_BATCH
-#define ELY_RECOVER_BATCH ELY_Q_BATCH  // recover register path: vectors per lane per load batch (0: all)
+#define ELY_RECOVER_BATCH 1  // recover register path: vectors per lane per load batch (0: all)
 #endif
 #ifndef ELY_RECOVER_WHOLE_VPL
 #define ELY_RECOVER_WHOLE_VPL 8  // recover register path: rows of this many vectors per lane or more load at once
@@ -111,29 +114,36 @@ constexpr int kFastK = 110;                    // |k| bound of the instruction p
 #define ELY_FP8_NT 3  // bit 0: nontemporal codec loads, bit 1: nontemporal stores
 #endif
 
+// Vector accesses carry no alignment beyond the element's: gfx950 loads and
+// stores 8- and 16-byte vectors at any address with the same instructions
+// (a probe of the quantize's and the dequantize's streams over 200 MB, at
+// 2- and 1-byte offsets against aligned: 7.70-7.94 against 8.10 TB/s, 6.22-
+// 6.53 against 6.86; nontemporal 5.40-5.83 against 6.75, 5.22-5.53 against
+// 6.27), so rows of any width take the vector paths.
 // Stores of streamed data; nontemporal when bit 1 of ELY_FP8_NT is set.
-typedef uint32_t ev4u __attribute__((ext_vector_type(4)));
-typedef uint32_t ev2u __attribute__((ext_vector_type(2)));
+typedef uint32_t ev4u __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t ev2u __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t ev1u __attribute__((aligned(1)));
 #define ELY_G1 __attribute__((address_space(1)))
 __device__ __forceinline__ void st_vec(void* p, uint4 v) {
 #if ELY_FP8_NT & 2
     __builtin_nontemporal_store(ev4u{v.x, v.y, v.z, v.w}, (ELY_G1 ev4u*)p);
 #else
-    *static_cast<uint4*>(p) = v;
+    *(ELY_G1 ev4u*)p = ev4u{v.x, v.y, v.z, v.w};
 #endif
 }
 __device__ __forceinline__ void st_vec2(void* p, uint2 v) {
 #if ELY_FP8_NT & 2
     __builtin_nontemporal_store(ev2u{v.x, v.y}, (ELY_G1 ev2u*)p);
 #else
-    *static_cast<uint2*>(p) = v;
+    *(ELY_G1 ev2u*)p = ev2u{v.x, v.y};
 #endif
 }
 __device__ __forceinline__ void st_u32(void* p, uint32_t v) {
 #if ELY_FP8_NT & 2
-    __builtin_nontemporal_store(v, (ELY_G1 uint32_t*)p);
+    __builtin_nontemporal_store(v, (ELY_G1 ev1u*)p);
 #else
-    *static_cast<uint32_t*>(p) = v;
+    *(ELY_G1 ev1u*)p = v;
 #endif
 }
 
@@ -143,26 +153,25 @@ __device__ __forceinline__ uint2 ld_vec2(const void* p) {
     const ev2u v = __builtin_nontemporal_load((const ELY_G1 ev2u*)p);
     return make_uint2(v[0], v[1]);
 #else
-    return *static_cast<const uint2*>(p);
+    const ev2u v = *(const ELY_G1 ev2u*)p;
+    return make_uint2(v[0], v[1]);
 #endif
 }
 __device__ __forceinline__ uint32_t ld_u32(const void* p) {
 #if ELY_FP8_NT & 1
-    return __builtin_nontemporal_load((const ELY_G1 uint32_t*)p);
+    return __builtin_nontemporal_load((const ELY_G1 ev1u*)p);
 #else
-    return *static_cast<const uint32_t*>(p);
+    return *(const ELY_G1 ev1u*)p;
 #endif
 }
 
 // One 16-byte load of streamed data.
 template <bool NT = (ELY_FP8_NT & 1) != 0>
-__device__ __forceinline__ uint4 ld_vec(const uint4* p) {
-    if (NT) {
-        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-        const v4u v = __builtin_nontemporal_load((const __attribute__((address_space(1))) v4u*)(const void*)p);
-        return make_uint4(v[0], v[1], v[2], v[3]);
-    }
-    return *p;
+__device__ __forceinline__ uint4 ld_vec(const void* p) {
+    ev4u v;
+    if (NT) v = __builtin_nontemporal_load((const ELY_G1 ev4u*)p);
+    else v = *(const ELY_G1 ev4u*)p;
+    return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
 template <bool BF16>
@@ -322,6 +331,36 @@ __device__ __forceinline__ void quant_slow(const void* x, int64_t base, int64_t 
 
 // ------------------------------------------------- wave-per-row (registers)
 
+// A row's vectors: vector i covers elements [i * EPV, i * EPV + EPV), the last
+// one of a row that is no whole number of vectors the row's last EPV elements
+// (it overlaps the vector before it: both write the same codes there), so a
+// row of any width >= EPV is whole vectors with no tail.  row_vec_off gives
+// the first element of lane-vector i, clamped to the last vector (lanes past
+// the row's end read that again, which no maximum notices).
+__device__ __forceinline__ int row_vec_off(int i, int epv, int cols) { return min(i * epv, cols - epv); }
+
+// The codes (and, with orow, the round trip's values) of a row's vectors
+// first + lane + kWave * j held in buf.
+template <int FMT, bool BF16, int VPL>
+__device__ __forceinline__ void store_row_vecs(const uint4 (&buf)[VPL], int first, int cols, const RowScale& rs,
+                                               uint8_t* qr, char* orow) {
+    constexpr int EPV = BF16 ? 8 : 4;
+    constexpr int ESZ = BF16 ? 2 : 4;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+        const int vi = first + kWave * j;
+        if (vi * EPV < cols) {
+            const int off = row_vec_off(vi, EPV, cols);
+            uint32_t words[2];
+            quant_vec_fast<FMT, BF16>(buf[j], rs, words, orow ? orow + off * ESZ : nullptr);
+            if (qr) {
+                if (BF16) st_vec2(qr + off, make_uint2(words[0], words[1]));
+                else st_u32(qr + off, words[0]);
+            }
+        }
+    }
+}
+
 template <int FMT, bool BF16, int VPL>
 __global__ __launch_bounds__(kQBlock) void quant_rows_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
                                                              uint8_t* __restrict__ q, int32_t* __restrict__ k,
@@ -331,48 +370,21 @@ __global__ __launch_bounds__(kQBlock) void quant_rows_kernel(const void* __restr
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t row = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     if (row >= rows) return;  // whole waves leave; the kernel has no block barrier
-    const int64_t nvec = cols / EPV;
-    const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + row * cols * ESZ);
-    // the row's loads go out in batches of QB vectors per lane, each batch's
-    // loads back to back: lanes past the row's end load its last vector (in
-    // bounds) and zero it afterwards
-    constexpr int QB = (ELY_Q_BATCH <= 0 || ELY_Q_BATCH > VPL) ? VPL : ELY_Q_BATCH;
+    const int c = (int)cols;
+    const char* xr = static_cast<const char*>(x) + row * cols * ESZ;
+    // every load of the row is issued before the first is waited for
     uint4 buf[VPL];
     uint32_t amax = 0;
 #pragma unroll
-    for (int j0 = 0; j0 < VPL; j0 += QB) {
+    for (int j = 0; j < VPL; ++j) buf[j] = ld_vec(xr + row_vec_off(lane + kWave * j, EPV, c) * ESZ);
 #pragma unroll
-        for (int j = j0; j < j0 + QB && j < VPL; ++j) {
-            const int64_t vi = lane + (int64_t)kWave * j;
-            buf[j] = ld_vec(xr + (vi < nvec ? vi : nvec - 1));
-        }
-#pragma unroll
-        for (int j = j0; j < j0 + QB && j < VPL; ++j) {
-            const int64_t vi = lane + (int64_t)kWave * j;
-            if (vi >= nvec) buf[j] = make_uint4(0u, 0u, 0u, 0u);
-            amax = vec_absmax<BF16>(buf[j], amax);
-        }
-        // the next batch is issued only once this one has arrived
-        if (QB < VPL) __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int j = 0; j < VPL; ++j) amax = vec_absmax<BF16>(buf[j], amax);
     amax = wave_max_u32(amax);
     const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(amax), BF16, BF16);
     if (lane == 0 && k) k[row] = rs.k;
     if (!rs.fast) return quant_slow<FMT, BF16>(x, row * cols, 0, cols, rs, q, out, lane);
-    uint8_t* qr = q ? q + row * cols : nullptr;
-    char* orow = out ? static_cast<char*>(out) + row * cols * ESZ : nullptr;
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        const int64_t vi = lane + (int64_t)kWave * j;
-        if (vi < nvec) {
-            uint32_t words[2];
-            quant_vec_fast<FMT, BF16>(buf[j], rs, words, orow ? orow + vi * 16 : nullptr);
-            if (qr) {
-                if (BF16) st_vec2(qr + vi * 8, make_uint2(words[0], words[1]));
-                else st_u32(qr + vi * 4, words[0]);
-            }
-        }
-    }
+    store_row_vecs<FMT, BF16, VPL>(buf, lane, c, rs, q ? q + row * cols : nullptr,
+                                   out ? static_cast<char*>(out) + row * cols * ESZ : nullptr);
 }
 
 // Long rows: the block's waves share one row, each wave a contiguous run of
@@ -385,31 +397,19 @@ __global__ __launch_bounds__(kRowBlock) void quant_block_row_kernel(const void* 
                                                                   void* __restrict__ out) {
     constexpr int EPV = BF16 ? 8 : 4;
     constexpr int ESZ = BF16 ? 2 : 4;
-    constexpr int QB = (ELY_Q_BATCH <= 0 || ELY_Q_BATCH > VPLW) ? VPLW : ELY_Q_BATCH;
     __shared__ uint32_t wmax[kRowWaves];
     const int lane = threadIdx.x & (kWave - 1);
     const int w = wave_uniform(threadIdx.x / kWave);
     const int64_t row = blockIdx.x;
-    const int64_t nvec = cols / EPV;
-    const int64_t v0 = (int64_t)w * kWave * VPLW;
-    const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + row * cols * ESZ);
+    const int c = (int)cols;
+    const int v0 = w * kWave * VPLW;
+    const char* xr = static_cast<const char*>(x) + row * cols * ESZ;
     uint4 buf[VPLW];
     uint32_t amax = 0;
 #pragma unroll
-    for (int j0 = 0; j0 < VPLW; j0 += QB) {
+    for (int j = 0; j < VPLW; ++j) buf[j] = ld_vec(xr + row_vec_off(v0 + lane + kWave * j, EPV, c) * ESZ);
 #pragma unroll
-        for (int j = j0; j < j0 + QB && j < VPLW; ++j) {
-            const int64_t vi = v0 + lane + (int64_t)kWave * j;
-            buf[j] = ld_vec(xr + (vi < nvec ? vi : nvec - 1));
-        }
-#pragma unroll
-        for (int j = j0; j < j0 + QB && j < VPLW; ++j) {
-            const int64_t vi = v0 + lane + (int64_t)kWave * j;
-            if (vi >= nvec) buf[j] = make_uint4(0u, 0u, 0u, 0u);
-            amax = vec_absmax<BF16>(buf[j], amax);
-        }
-        if (QB < VPLW) __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int j = 0; j < VPLW; ++j) amax = vec_absmax<BF16>(buf[j], amax);
     amax = wave_max_u32(amax);
     if (lane == 0) wmax[w] = amax;
     __syncthreads();
@@ -419,23 +419,11 @@ __global__ __launch_bounds__(kRowBlock) void quant_block_row_kernel(const void* 
     const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(amax), BF16, BF16);
     if (threadIdx.x == 0 && k) k[row] = rs.k;
     if (!rs.fast) {
-        const int64_t e0 = min(v0 * EPV, cols), e1 = min((v0 + (int64_t)kWave * VPLW) * EPV, cols);
+        const int64_t e0 = min((int64_t)v0 * EPV, cols), e1 = min((int64_t)(v0 + kWave * VPLW) * EPV, cols);
         return quant_slow<FMT, BF16>(x, row * cols, e0, e1, rs, q, out, lane);
     }
-    uint8_t* qr = q ? q + row * cols : nullptr;
-    char* orow = out ? static_cast<char*>(out) + row * cols * ESZ : nullptr;
-#pragma unroll
-    for (int j = 0; j < VPLW; ++j) {
-        const int64_t vi = v0 + lane + (int64_t)kWave * j;
-        if (vi < nvec) {
-            uint32_t words[2];
-            quant_vec_fast<FMT, BF16>(buf[j], rs, words, orow ? orow + vi * 16 : nullptr);
-            if (qr) {
-                if (BF16) st_vec2(qr + vi * 8, make_uint2(words[0], words[1]));
-                else st_u32(qr + vi * 4, words[0]);
-            }
-        }
-    }
+    store_row_vecs<FMT, BF16, VPLW>(buf, v0 + lane, c, rs, q ? q + row * cols : nullptr,
+                                    out ? static_cast<char*>(out) + row * cols * ESZ : nullptr);
 }
 
 // ------------------------------------------------------- split long rows
@@ -773,18 +761,58 @@ __global__ __launch_bounds__(kQBlock) void quant_hint_fixup_kernel(const void* _
 
 // -------------------------------------------------------------- dequantize
 
-// Codes in rows whose length is a multiple of 16 (and 16-byte aligned
-// buffers) are dequantized as one flat array: wave w takes codes
+// The codes are dequantized as one flat array: wave w takes codes
 // [S w, S w + S) (S = kDeqSegCodes), which may span rows.  A lane takes CPL
 // codes per step (8 for bf16 output, 4 for fp32), so that each store
 // instruction of a wave writes one contiguous 1 KB run; every lane issues
 // its loads (all of them, or batches of ELY_DEQ_BATCH) before the first is
-// used, and each CPL-code vector lies in one row.  Rows at least a segment
+// used.  When rows are whole vectors (a multiple of 16 codes, 16-byte
+// aligned buffers) each CPL-code vector lies in one row; RAGGED takes rows of
+// any width >= CPL at any alignment, where a vector may hold the end of one
+// row and the start of the next (`cut` codes of it in the first) and the
+// array's last vector is its last CPL codes.  Rows at least a segment
 // wide give a segment at most two exponents, read once per wave (C1 back to
 // back: 5.89-5.94 TB/s against 5.76-5.80 with a division and an exponent
 // load per vector); narrower rows look theirs up per vector.  Short
 // segments (many short-lived waves) measured fastest.
-template <int FMT, bool BF16OUT, bool IDX32>
+
+// CPL codes at e, the first `cut` of them of a row with exponent k1, the rest
+// of the next row's k2.
+template <int FMT, bool BF16OUT, int CPL>
+__device__ __forceinline__ void dequant_two_rows(const uint32_t (&w)[CPL / 4], int k1, int k2, int cut, void* out,
+                                                 int64_t e) {
+    if (k1 >= -kFastK && k1 <= kFastK && k2 >= -kFastK && k2 <= kFastK) {
+        const float s1 = __uint_as_float((uint32_t)(127 + k1) << 23), s2 = __uint_as_float((uint32_t)(127 + k2) << 23);
+        float o[CPL];
+#pragma unroll
+        for (int h = 0; h < CPL / 4; ++h) {
+            cvt_pk_f32<FMT, false>(w[h], o[4 * h], o[4 * h + 1]);
+            cvt_pk_f32<FMT, true>(w[h], o[4 * h + 2], o[4 * h + 3]);
+        }
+        uint32_t b[CPL];
+#pragma unroll
+        for (int t = 0; t < CPL; ++t) {
+            const float v = o[t] * (t < cut ? s1 : s2);
+            b[t] = BF16OUT ? (v != v ? 0x7FC0u : fast_bf16_bits(v)) : __float_as_uint(v);
+        }
+        if (BF16OUT)
+            st_vec(static_cast<uint16_t*>(out) + e,
+                   make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[CPL - 4] | (b[CPL - 3] << 16),
+                              b[CPL - 2] | (b[CPL - 1] << 16)));
+        else
+            st_vec(static_cast<float*>(out) + e, make_uint4(b[0], b[1], b[2], b[3]));
+        return;
+    }
+    const float s1 = pow2_dtype(k1, BF16OUT), s2 = pow2_dtype(k2, BF16OUT);
+#pragma unroll 1
+    for (int t = 0; t < CPL; ++t) {
+        const float o = dequant_sw<FMT, BF16OUT>((w[t / 4] >> (8 * (t % 4))) & 0xFFu, t < cut ? s1 : s2);
+        if (BF16OUT) static_cast<uint16_t*>(out)[e + t] = (uint16_t)f32_to_bf16(o);
+        else static_cast<float*>(out)[e + t] = o;
+    }
+}
+
+template <int FMT, bool BF16OUT, bool IDX32, bool RAGGED>
 __global__ __launch_bounds__(kQBlock) void dequant_flat_kernel(const uint8_t* __restrict__ q,
                                                                const int32_t* __restrict__ k, int64_t n,
                                                                int64_t cols, void* __restrict__ out) {
@@ -794,7 +822,7 @@ __global__ __launch_bounds__(kQBlock) void dequant_flat_kernel(const uint8_t* __
     const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     const int64_t e0 = gw * kDeqSegCodes;
     if (e0 >= n) return;
-    const int64_t nv = min(kDeqSegCodes, n - e0) / CPL;
+    const int64_t nv = (min(kDeqSegCodes, n - e0) + (RAGGED ? CPL - 1 : 0)) / CPL;
     constexpr int DB = (ELY_DEQ_BATCH <= 0 || ELY_DEQ_BATCH > VPL) ? VPL : ELY_DEQ_BATCH;
     // rows at least a segment wide: the segment meets at most two rows, the
     // one holding code e0 and, from code `split` on, the next; the wave reads
@@ -808,7 +836,8 @@ __global__ __launch_bounds__(kQBlock) void dequant_flat_kernel(const uint8_t* __
 #pragma unroll
         for (int j = j0; j < j0 + DB && j < VPL; ++j) {
             const int64_t vi = lane + (int64_t)kWave * j;
-            const uint8_t* src = q + e0 + (vi < nv ? vi : nv - 1) * CPL;
+            const int64_t ev = e0 + (vi < nv ? vi : nv - 1) * CPL;
+            const uint8_t* src = q + (RAGGED ? min(ev, n - CPL) : ev);
             if (CPL == 8) {
                 const uint2 w = ld_vec2(src);
                 buf[j][0] = w.x;
@@ -820,7 +849,9 @@ __global__ __launch_bounds__(kQBlock) void dequant_flat_kernel(const uint8_t* __
         // the exponents are read once the first codes are requested: a wait
         // for these loads ahead of the code loads would hold those back
         if (j0 == 0 && two_rows) {
-            const int64_t row0 = IDX32 ? (int64_t)((uint32_t)e0 / (uint32_t)cols) : e0 / cols;
+            // a segment shorter than a vector is the array's last vector, which begins before it
+            const int64_t es = RAGGED ? min(e0, n - CPL) : e0;
+            const int64_t row0 = IDX32 ? (int64_t)((uint32_t)es / (uint32_t)cols) : es / cols;
             split = (row0 + 1) * cols;
             k_lo = k[row0];
             k_hi = k[split < n ? row0 + 1 : row0];
@@ -829,13 +860,25 @@ __global__ __launch_bounds__(kQBlock) void dequant_flat_kernel(const uint8_t* __
         for (int j = j0; j < j0 + DB && j < VPL; ++j) {
             const int64_t vi = lane + (int64_t)kWave * j;
             if (vi >= nv) continue;
-            const int64_t e = e0 + vi * CPL;
-            int kk;
+            const int64_t e = RAGGED ? min(e0 + vi * CPL, n - CPL) : e0 + vi * CPL;
+            int kk, kk2 = 0, cut = CPL;
             if (two_rows) {
                 kk = e < split ? k_lo : k_hi;
+                if (RAGGED && e < split && e + CPL > split) {
+                    cut = (int)(split - e);
+                    kk2 = k_hi;
+                }
             } else {
                 const int64_t row = IDX32 ? (int64_t)((uint32_t)e / (uint32_t)cols) : e / cols;
                 kk = k[row];
+                if (RAGGED && e + CPL > (row + 1) * cols) {
+                    cut = (int)((row + 1) * cols - e);
+                    kk2 = k[row + 1];
+                }
+            }
+            if (RAGGED && cut < CPL && kk2 != kk) {
+                dequant_two_rows<FMT, BF16OUT, CPL>(buf[j], kk, kk2, cut, out, e);
+                continue;
             }
             if (kk >= -kFastK && kk <= kFastK) {
                 const float s_up = __uint_as_float((uint32_t)(127 + kk) << 23);
@@ -1364,17 +1407,28 @@ static void dispatch_rows(int vpl, const void* x, int64_t rows, int64_t cols, ui
     }
 }
 
-// Register path's vectors per lane for these columns, or 0 when the row does
-// not fit it.
-static int rows_vpl(int64_t cols, int32_t dtype, const void* x, const uint8_t* q, const void* out) {
+// Whether these rows are whole 16-byte vectors at aligned addresses.
+static bool whole_vecs(int64_t cols, int32_t dtype, const void* x, const uint8_t* q, const void* out) {
     const int64_t epv = dtype == ELY_BF16 ? 8 : 4;
-    if (cols == 0 || cols % epv != 0) return 0;
-    if (!aligned16(x) || (out && !aligned16(out))) return 0;
-    if (q && (reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv) != 0) return 0;
-    const int64_t nvec = cols / epv;
+    return cols % epv == 0 && aligned16(x) && (!out || aligned16(out)) &&
+           (!q || reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv == 0);
+}
+
+// Register path's vectors per lane for these columns, or 0 when the row does
+// not fit it: any row of at least one vector, at any element's alignment.
+static int rows_vpl(int64_t cols, int32_t dtype, const void* x, const void* out) {
+    const int64_t epv = dtype == ELY_BF16 ? 8 : 4, esz = dtype == ELY_BF16 ? 2 : 4;
+    if (cols < epv || reinterpret_cast<uintptr_t>(x) % esz || reinterpret_cast<uintptr_t>(out) % esz) return 0;
+    const int64_t nvec = (cols + epv - 1) / epv;
     for (int v : kVplChoices)
         if (nvec <= (int64_t)kWave * v) return v;
     return 0;
+}
+
+// The shapes whose calls carry the split path's workspace: rows that are not
+// whole aligned vectors or are longer than the register paths.
+static bool wants_workspace(int64_t cols, int32_t dtype, const void* x, const uint8_t* q, const void* out) {
+    return !whole_vecs(cols, dtype, x, q, out) || rows_vpl(cols, dtype, x, out) == 0;
 }
 
 // Row maxima, then the partial maxima (at most max(rows, kSplitWaves) of them).
@@ -1422,7 +1476,17 @@ static void quantize_impl(const void* x, int64_t rows, int64_t cols, uint8_t* q,
         return;
     }
     const int32_t dt = BF16 ? ELY_BF16 : ELY_F32;
-    const int vpl = rows_vpl(cols, dt, x, q, out);
+    const int vec = whole_vecs(cols, dt, x, q, out);
+    const bool want_ws = wants_workspace(cols, dt, x, q, out);
+    const bool guess = want_ws && allow_guess && rows == 1 && (q || out) && vec &&
+                       cols >= ((int64_t)ELY_GUESS_MIN_MB << 20) / (BF16 ? 2 : 4) && workspace &&
+                       ws_bytes >= (int64_t)guess_ws_bytes(cols);
+    if (want_ws && !guess && (!workspace || ws_bytes < (int64_t)split_ws_bytes(rows)))
+        fail(ELY_EWORKSPACE, "fp8 quantize: this shape needs " + std::to_string(split_ws_bytes(rows)) +
+                                 " workspace bytes (ely_fp8_workspace_bytes)");
+    int vpl = rows_vpl(cols, dt, x, out);
+    // a block per row counts its threads in 32 bits; the split path's waves take more rows
+    if (want_ws && vpl > kMaxWaveVpl && rows > 0xFFFFFFFFLL / kRowBlock) vpl = 0;
     if (vpl > kMaxWaveVpl) {
         // one block per row: kRowWaves waves of ceil(vpl / kRowWaves) vectors per lane
         if (rows > 0xFFFFFFFFLL / kRowBlock) fail(ELY_EINVAL, "fp8 quantize: too many rows for one launch");
@@ -1436,15 +1500,7 @@ static void quantize_impl(const void* x, int64_t rows, int64_t cols, uint8_t* q,
         return;
     }
     if (vpl) return dispatch_rows<FMT, BF16>(vpl, x, rows, cols, q, k, out, s);
-    const int64_t epv = BF16 ? 8 : 4;
-    const int vec = (cols % epv == 0) && aligned16(x) && (!out || aligned16(out)) &&
-                    (!q || reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv == 0);
-    if (allow_guess && rows == 1 && (q || out) && vec && cols >= ((int64_t)ELY_GUESS_MIN_MB << 20) / (BF16 ? 2 : 4) &&
-        workspace && ws_bytes >= (int64_t)guess_ws_bytes(cols))
-        return quantize_guess_impl<FMT, BF16>(x, cols, q, k, out, workspace, ws_bytes, s);
-    if (!workspace || ws_bytes < (int64_t)split_ws_bytes(rows))
-        fail(ELY_EWORKSPACE, "fp8 quantize: this shape needs " + std::to_string(split_ws_bytes(rows)) +
-                                 " workspace bytes (ely_fp8_workspace_bytes)");
+    if (guess) return quantize_guess_impl<FMT, BF16>(x, cols, q, k, out, workspace, ws_bytes, s);
     uint32_t* rowmax = static_cast<uint32_t*>(workspace);
     const int64_t segs = (cols + kSegElems - 1) / kSegElems;
     if (rows > INT64_MAX / segs) fail(ELY_EINVAL, "too many segments");
@@ -1470,9 +1526,7 @@ static void quantize_hint_impl(const void* x, int64_t n, int32_t k_hint, const i
     if (!workspace || ws_bytes < (int64_t)hint_ws_bytes(n))
         fail(ELY_EWORKSPACE, "ely_fp8_quantize_hint: workspace of " + std::to_string(ws_bytes) + " bytes, need " +
                                  std::to_string(hint_ws_bytes(n)) + " (ely_fp8_hint_workspace_bytes)");
-    const int64_t epv = BF16 ? 8 : 4;
-    const bool vec = n > 0 && n % epv == 0 && aligned16(x) && (!out || aligned16(out)) &&
-                     (!q || reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv == 0);
+    const bool vec = n > 0 && whole_vecs(n, BF16 ? ELY_BF16 : ELY_F32, x, q, out);
     if (!vec || (!k_hint_dev && (k_hint < -kFastK || k_hint > kFastK))) {
         // no one-pass form for this tensor or hint: the split path, a miss
         quantize_impl<FMT, BF16>(x, 1, n, q, k, out, workspace, ws_bytes, s, false);
@@ -1528,26 +1582,33 @@ static void quantize_guess_impl(const void* x, int64_t n, uint8_t* q, int32_t* k
                                   ws_bytes, s, true);
 }
 
+template <int FMT, bool BF16OUT, bool RAGGED>
+static void launch_dequant_flat(const uint8_t* q, const int32_t* k, int64_t n, int64_t cols, void* out, hipStream_t s) {
+    const unsigned blocks = blocks_for_waves((n + kDeqSegCodes - 1) / kDeqSegCodes);
+    if (n < ((int64_t)1 << 32))
+        hipLaunchKernelGGL((dequant_flat_kernel<FMT, BF16OUT, true, RAGGED>), dim3(blocks), dim3(kQBlock), ELY_DEQ_LDS, s, q,
+                           k, n, cols, out);
+    else
+        hipLaunchKernelGGL((dequant_flat_kernel<FMT, BF16OUT, false, RAGGED>), dim3(blocks), dim3(kQBlock), ELY_DEQ_LDS, s, q,
+                           k, n, cols, out);
+    check_launch("dequant_flat_kernel");
+}
+
 template <int FMT, bool BF16OUT>
 static void dequantize_impl(const uint8_t* q, const int32_t* k, int64_t rows, int64_t cols, void* out,
                             hipStream_t s) {
     if (rows == 0 || cols == 0) return;
-    if ((cols % 16 == 0) && aligned16(q) && aligned16(out)) {
-        const int64_t n = rows * cols;
-        const unsigned blocks = blocks_for_waves((n + kDeqSegCodes - 1) / kDeqSegCodes);
-        if (n < ((int64_t)1 << 32))
-            hipLaunchKernelGGL((dequant_flat_kernel<FMT, BF16OUT, true>), dim3(blocks), dim3(kQBlock), ELY_DEQ_LDS, s, q, k, n,
-                               cols, out);
-        else
-            hipLaunchKernelGGL((dequant_flat_kernel<FMT, BF16OUT, false>), dim3(blocks), dim3(kQBlock), ELY_DEQ_LDS, s, q, k, n,
-                               cols, out);
-        check_launch("dequant_flat_kernel");
-        return;
-    }
+    const int64_t n = rows * cols;
+    if ((cols % 16 == 0) && aligned16(q) && aligned16(out))
+        return launch_dequant_flat<FMT, BF16OUT, false>(q, k, n, cols, out, s);
     const int64_t segs = (cols + kDeqSegCodes - 1) / kDeqSegCodes;
     if (rows > INT64_MAX / segs) fail(ELY_EINVAL, "too many segments");
-    hipLaunchKernelGGL((dequant_any_kernel<FMT, BF16OUT>), dim3(blocks_for_waves(rows * segs)), dim3(kQBlock), 0, s, q,
-                       k, rows, cols, segs, out);
+    const unsigned any_blocks = blocks_for_waves(rows * segs);
+    // rows of at least a vector (a vector then meets at most two rows)
+    if (cols >= 8 && reinterpret_cast<uintptr_t>(out) % (BF16OUT ? 2 : 4) == 0)
+        return launch_dequant_flat<FMT, BF16OUT, true>(q, k, n, cols, out, s);
+    hipLaunchKernelGGL((dequant_any_kernel<FMT, BF16OUT>), dim3(any_blocks), dim3(kQBlock), 0, s, q, k, rows, cols, segs,
+                       out);
     check_launch("dequant_any_kernel");
 }
 
@@ -1734,7 +1795,7 @@ int ely_fp8_quantize_noalloc(const void* x, int32_t x_dtype, int64_t rows, int64
         // its row maxima and partials must fit the static array.  Every
         // scratch word the split launches read was written by an earlier
         // launch of the same call, so nothing needs clearing between calls.
-        const bool split = rows > 0 && cols > 0 && rows_vpl(cols, x_dtype, x, q, nullptr) == 0;
+        const bool split = rows > 0 && cols > 0 && wants_workspace(cols, x_dtype, x, q, nullptr);
         void* ws = nullptr;
         if (split) {
             const size_t need = split_ws_bytes(rows);

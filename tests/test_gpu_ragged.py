@@ -1,0 +1,75 @@
+"""Shapes that are no whole number of 16-byte vectors, and addresses off a
+16-byte boundary, on the vector paths: every byte against the oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import activation, bits, f32_equal, say
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "bf16": torch.bfloat16}
+
+
+def _codec_equals_the_oracle(oracle, x, fmt):
+    from elysium_wan_amd import fp8
+
+    raw = bits(x) if x.dtype == torch.bfloat16 else bits(x).astype(np.float32)
+    name = "bf16" if x.dtype == torch.bfloat16 else "f32"
+    same = np.array_equal if name == "bf16" else f32_equal
+    q, k = fp8.quantize(x, fmt)
+    oq, ok = oracle.quantize(raw, fmt)
+    assert np.array_equal(bits(k).reshape(-1), ok.reshape(-1)), "exponents"
+    assert np.array_equal(bits(q).reshape(-1), oq.reshape(-1)), "fp8 bytes"
+    assert same(bits(fp8.roundtrip(x, fmt)).reshape(-1), oracle.roundtrip(raw, fmt).reshape(-1)), "round trip"
+    for out in ("f32", "bf16"):
+        got, want = bits(fp8.dequantize(q, k, DT[out])).reshape(-1), oracle.dequantize(oq, ok, fmt, out).reshape(-1)
+        assert (np.array_equal if out == "bf16" else f32_equal)(got, want), f"dequantize {out}"
+
+
+# one vector and its neighbours, a lane's and a wave's last vector, the edges
+# of each kernel's row lengths, and rows past the registers
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("dname", ["bf16", "f32"])
+@pytest.mark.parametrize("cols", [3, 4, 5, 7, 8, 9, 15, 17, 255, 511, 513, 1023, 1025, 1601, 3071, 3073, 4095, 4097, 8191, 8193])
+def test_rows_of_any_width_equal_the_oracle(oracle, fmt, dname, cols):
+    rows = 9 + 2048 // cols
+    base = activation((rows * cols + 3,), seed=cols % 89, dtype=DT[dname])
+    for off in (0, 1, 3):  # elements off the allocation's boundary
+        x = base[off : off + rows * cols].reshape(rows, cols).clone() if off == 0 else base[off : off + rows * cols].reshape(rows, cols)
+        if off == 1:  # rows outside the instruction path beside rows inside it
+            x[1] = 0.0
+            x[2, cols - 1] = float("nan")
+            x[3, cols // 2] = float("-inf")
+            x[4] *= 2.0**-120
+            x[5] *= 2.0**115
+        say("fp8 ragged rows", fmt, dname, rows, cols, "offset", off)
+        _codec_equals_the_oracle(oracle, x, fmt)
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("cols", [8, 9, 13, 100, 1000, 1025, 1601, 2053])
+def test_ragged_dequantize_with_a_distinct_exponent_per_row(oracle, fmt, cols):
+    """Every code, neighbouring rows' exponents different and some outside
+    the instruction path, so that a vector holding the end of one row and the
+    start of the next shows a wrong one; q off its boundary too."""
+    from elysium_wan_amd import fp8
+
+    rows = max(3, (5 * 1024 + 7) // cols)
+    rng = np.random.default_rng(cols)
+    codes = ((np.arange(rows * cols, dtype=np.int64) * 37 + 11) % 256).astype(np.uint8)
+    kk = rng.integers(-140, 141, rows).astype(np.int32)
+    kk[1:][kk[1:] == kk[:-1]] += 1
+    for off in (0, 1):
+        buf = torch.empty(rows * cols + off, dtype=torch.uint8, device="cuda")
+        buf[off:] = torch.from_numpy(codes).cuda()
+        q = buf[off:].view(fp8.FORMATS[fmt][0]).reshape(rows, cols)
+        k = torch.from_numpy(kk.reshape(rows, 1)).cuda()
+        for out in ("f32", "bf16"):
+            say("fp8 ragged dequantize", fmt, cols, out, "offset", off)
+            d = bits(fp8.dequantize(q, k, DT[out])).reshape(-1)
+            od = oracle.dequantize(codes.reshape(rows, cols), kk, fmt, out).reshape(-1)
+            assert f32_equal(d, od) if out == "f32" else np.array_equal(d, od)
