@@ -2,14 +2,14 @@
 //
 // quantize (fp8.py:28-49): per row, k = frexp(amax|x|).exponent - ebias and
 // q = fp8(x * 2^-k).  Three launch shapes:
-//   * rows that fit registers (one vector up to 64 lanes x 16 vectors of 16
-//     bytes: 8 to 8192 bf16 / 4 to 4096 fp32 columns, any width and any
-//     element's alignment): the row is read once into VGPRs, |x|max is a
+//   * rows that fit registers (one vector up to 16 waves x 64 lanes x 4
+//     vectors of 16 bytes: 8 to 32,768 bf16 / 4 to 16,384 fp32 columns, any
+//     width and any element's alignment): the row is read once into VGPRs, |x|max is a
 //     butterfly over the wave, and codes are written from the same
 //     registers: one HBM read and one write per element (3 B/elem for bf16
 //     -> fp8).  Rows of up to 6 vectors per lane take one wave; longer ones
-//     are shared by a block's 4 waves, whose maxima meet in LDS, so that each
-//     wave holds at most 4 vectors and more rows stream at once.  A width
+//     are shared by a block's 4, 8 or 16 waves, whose maxima meet in LDS, so
+//     that each wave holds at most 4 vectors and more rows stream at once.  A width
 //     that is no whole number of vectors ends in a vector that overlaps the
 //     one before it: [16376, 1601] bf16 quantizes in 17 us where element
 //     loads with two reads of x took 65 (79 MB: 4.5 against 1.2 TB/s).
@@ -101,7 +101,7 @@ namespace ely {
 #endif
 constexpr int kQBlock = ELY_QBLOCK;            // threads per block; each wave takes its own row or segment
 constexpr int kWavesPerBlock = kQBlock / kWave;
-constexpr int kRowBlock = 256;                 // the block-row quantize and the row-max reduce: 4 waves share one row
+constexpr int kRowBlock = 256;                 // the row-max reduce: 4 waves share one row
 constexpr int kRowWaves = kRowBlock / kWave;
 constexpr int64_t kSegElems = 2048;            // split-path segment, elements
 constexpr int64_t kDeqSegCodes = ELY_DEQ_SEG;  // dequantize segment, codes
@@ -387,17 +387,17 @@ __global__ __launch_bounds__(kQBlock) void quant_rows_kernel(const void* __restr
                                    out ? static_cast<char*>(out) + row * cols * ESZ : nullptr);
 }
 
-// Long rows: the block's waves share one row, each wave a contiguous run of
+// Long rows: the block's W waves share one row, each wave a contiguous run of
 // kWave * VPLW vectors; the waves' |x|max meet in LDS across one barrier.
 // The host launches exactly one block per row, so every wave of a block
 // reaches the barrier.
-template <int FMT, bool BF16, int VPLW>
-__global__ __launch_bounds__(kRowBlock) void quant_block_row_kernel(const void* __restrict__ x, int64_t cols,
+template <int FMT, bool BF16, int W, int VPLW>
+__global__ __launch_bounds__(W * kWave) void quant_block_row_kernel(const void* __restrict__ x, int64_t cols,
                                                                   uint8_t* __restrict__ q, int32_t* __restrict__ k,
                                                                   void* __restrict__ out) {
     constexpr int EPV = BF16 ? 8 : 4;
     constexpr int ESZ = BF16 ? 2 : 4;
-    __shared__ uint32_t wmax[kRowWaves];
+    __shared__ uint32_t wmax[W];
     const int lane = threadIdx.x & (kWave - 1);
     const int w = wave_uniform(threadIdx.x / kWave);
     const int64_t row = blockIdx.x;
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(kRowBlock) void quant_block_row_kernel(const void* 
     __syncthreads();
     amax = wmax[0];
 #pragma unroll
-    for (int i = 1; i < kRowWaves; ++i) amax = max(amax, wmax[i]);
+    for (int i = 1; i < W; ++i) amax = max(amax, wmax[i]);
     const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(amax), BF16, BF16);
     if (threadIdx.x == 0 && k) k[row] = rs.k;
     if (!rs.fast) {
@@ -1380,11 +1380,20 @@ static unsigned blocks_for_waves(int64_t waves) {
     return (unsigned)b;
 }
 
-// Vectors per lane of the register paths: a wave per row up to kMaxWaveVpl,
-// a block of kRowWaves waves per row above (the block's loads in flight
-// per row stay the same, and more rows stream at once).
-constexpr int kVplChoices[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+// The register paths, by a row's vectors in units of one per lane of a wave
+// (rows_units): a wave per row up to kMaxWaveVpl units, a block per row above,
+// of as many waves as keep at most 4 vectors per lane in each: 4 waves to 16
+// units, 8 to 32, 16 to kMaxRowUnits (32,768 bf16 or 16,384 fp32 columns).
+// Against the split path, which reads x twice and makes three launches:
+// [4096, 6144] fp32 quantizes in 21.2 us against 37.2 (5.9 against 3.4 TB/s),
+// [4096, 20480] bf16 in 43 against 66, [2048, 16384] fp32 in 28 against 50,
+// [2048, 32768] bf16 in 34 against 55, and one row of 32,768 bf16 in 4.2
+// against 10.8 (launch-bound).
 constexpr int kMaxWaveVpl = 6;
+constexpr int kMaxRowUnits = 64;
+// Longer rows than this, and rows that are not whole aligned vectors, are
+// called with the split path's workspace, whether it is used or not.
+constexpr int kNoWorkspaceUnits = 16;
 
 template <int FMT, bool BF16, int VPL>
 static void launch_rows(const void* x, int64_t rows, int64_t cols, uint8_t* q, int32_t* k, void* out, hipStream_t s) {
@@ -1414,21 +1423,33 @@ static bool whole_vecs(int64_t cols, int32_t dtype, const void* x, const uint8_t
            (!q || reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv == 0);
 }
 
-// Register path's vectors per lane for these columns, or 0 when the row does
-// not fit it: any row of at least one vector, at any element's alignment.
-static int rows_vpl(int64_t cols, int32_t dtype, const void* x, const void* out) {
+// A row's vectors in units of one per lane of a wave (kWave vectors), for any
+// row of at least one vector at any element's alignment that the register
+// paths take; 0 for the others.
+static int rows_units(int64_t cols, int32_t dtype, const void* x, const void* out) {
     const int64_t epv = dtype == ELY_BF16 ? 8 : 4, esz = dtype == ELY_BF16 ? 2 : 4;
     if (cols < epv || reinterpret_cast<uintptr_t>(x) % esz || reinterpret_cast<uintptr_t>(out) % esz) return 0;
-    const int64_t nvec = (cols + epv - 1) / epv;
-    for (int v : kVplChoices)
-        if (nvec <= (int64_t)kWave * v) return v;
-    return 0;
+    const int64_t per = epv * kWave;
+    return cols <= per * kMaxRowUnits ? (int)((cols + per - 1) / per) : 0;
 }
 
-// The shapes whose calls carry the split path's workspace: rows that are not
-// whole aligned vectors or are longer than the register paths.
+// The shapes whose calls carry the split path's workspace.
 static bool wants_workspace(int64_t cols, int32_t dtype, const void* x, const uint8_t* q, const void* out) {
-    return !whole_vecs(cols, dtype, x, q, out) || rows_vpl(cols, dtype, x, out) == 0;
+    const int units = rows_units(cols, dtype, x, out);
+    return !whole_vecs(cols, dtype, x, q, out) || units == 0 || units > kNoWorkspaceUnits;
+}
+
+template <int FMT, bool BF16, int W>
+static void launch_block_row(int units, const void* x, int64_t rows, int64_t cols, uint8_t* q, int32_t* k, void* out,
+                             hipStream_t s) {
+    const dim3 g((unsigned)rows), b(W * kWave);
+    switch ((units + W - 1) / W) {
+        case 2: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, W, 2>), g, b, 0, s, x, cols, q, k, out); break;
+        case 3: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, W, 3>), g, b, 0, s, x, cols, q, k, out); break;
+        case 4: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, W, 4>), g, b, 0, s, x, cols, q, k, out); break;
+        default: fail(ELY_EINVAL, "internal: no block-row path for this row length");
+    }
+    check_launch("quant_block_row_kernel");
 }
 
 // Row maxima, then the partial maxima (at most max(rows, kSplitWaves) of them).
@@ -1484,22 +1505,20 @@ static void quantize_impl(const void* x, int64_t rows, int64_t cols, uint8_t* q,
     if (want_ws && !guess && (!workspace || ws_bytes < (int64_t)split_ws_bytes(rows)))
         fail(ELY_EWORKSPACE, "fp8 quantize: this shape needs " + std::to_string(split_ws_bytes(rows)) +
                                  " workspace bytes (ely_fp8_workspace_bytes)");
-    int vpl = rows_vpl(cols, dt, x, out);
-    // a block per row counts its threads in 32 bits; the split path's waves take more rows
-    if (want_ws && vpl > kMaxWaveVpl && rows > 0xFFFFFFFFLL / kRowBlock) vpl = 0;
-    if (vpl > kMaxWaveVpl) {
-        // one block per row: kRowWaves waves of ceil(vpl / kRowWaves) vectors per lane
-        if (rows > 0xFFFFFFFFLL / kRowBlock) fail(ELY_EINVAL, "fp8 quantize: too many rows for one launch");
-        switch ((vpl + kRowWaves - 1) / kRowWaves) {
-            case 2: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, 2>), dim3((unsigned)rows), dim3(kRowBlock), 0, s, x, cols, q, k, out); break;
-            case 3: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, 3>), dim3((unsigned)rows), dim3(kRowBlock), 0, s, x, cols, q, k, out); break;
-            case 4: hipLaunchKernelGGL((quant_block_row_kernel<FMT, BF16, 4>), dim3((unsigned)rows), dim3(kRowBlock), 0, s, x, cols, q, k, out); break;
-            default: fail(ELY_EINVAL, "internal: no block-row path for this row length");
-        }
-        check_launch("quant_block_row_kernel");
-        return;
+    int units = rows_units(cols, dt, x, out);
+    if (units > kMaxWaveVpl) {
+        // one block per row; a dispatch counts its threads in 32 bits, and
+        // the split path's waves take more rows than that
+        const int waves = units <= 16 ? 4 : units <= 32 ? 8 : 16;
+        const bool fits = rows <= 0xFFFFFFFFLL / (waves * kWave);
+        if (!fits && !want_ws) fail(ELY_EINVAL, "fp8 quantize: too many rows for one launch");
+        if (fits)
+            return waves == 4 ? launch_block_row<FMT, BF16, 4>(units, x, rows, cols, q, k, out, s)
+                   : waves == 8 ? launch_block_row<FMT, BF16, 8>(units, x, rows, cols, q, k, out, s)
+                                : launch_block_row<FMT, BF16, 16>(units, x, rows, cols, q, k, out, s);
+    } else if (units) {
+        return dispatch_rows<FMT, BF16>(units, x, rows, cols, q, k, out, s);
     }
-    if (vpl) return dispatch_rows<FMT, BF16>(vpl, x, rows, cols, q, k, out, s);
     if (guess) return quantize_guess_impl<FMT, BF16>(x, cols, q, k, out, workspace, ws_bytes, s);
     uint32_t* rowmax = static_cast<uint32_t*>(workspace);
     const int64_t segs = (cols + kSegElems - 1) / kSegElems;

@@ -34,7 +34,7 @@ def _codec_equals_the_oracle(oracle, x, fmt):
 # of each kernel's row lengths, and rows past the registers
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
 @pytest.mark.parametrize("dname", ["bf16", "f32"])
-@pytest.mark.parametrize("cols", [3, 4, 5, 7, 8, 9, 15, 17, 255, 511, 513, 1023, 1025, 1601, 3071, 3073, 4095, 4097, 8191, 8193])
+@pytest.mark.parametrize("cols", [3, 4, 5, 7, 8, 9, 15, 17, 255, 511, 513, 1023, 1025, 1601, 3071, 3073, 4095, 4097, 8191, 8193, 12001, 16383, 16385, 24577, 32767, 32769])
 def test_rows_of_any_width_equal_the_oracle(oracle, fmt, dname, cols):
     rows = 9 + 2048 // cols
     base = activation((rows * cols + 3,), seed=cols % 89, dtype=DT[dname])
