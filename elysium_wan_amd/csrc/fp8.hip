@@ -17,12 +17,10 @@
 //     vector at a time took C1's round trip from 30.0 to 32.0 us).
 //   * longer rows (per-tensor scaling is rows = 1): the row is cut into
 //     2048-element segments.  A first launch reduces the row's |x|max into
-//     at most 2,048 partial maxima (each wave strides over its row's
-//     segments; integer max, so order-free), a small second launch folds the
-//     partials per row, a third converts one segment per wave.  Two reads
-//     of x, no atomics.
-//   * any other shape (longer rows that are no whole aligned vectors, rows
-//     shorter than a vector): the same launches with element-wise loads.
+//     at most 256 partial maxima (each wave strides over its row's segments;
+//     integer max, so order-free), a second converts one segment per wave,
+//     which folds the partials first.  Two reads of x, no atomics.
+//   * rows shorter than a vector: the same launches with element-wise loads.
 // Every row whose exponent keeps 2^-k, 2^k and every product exact
 // (|k| <= 110, finite |x|max) converts with the instructions: bf16 words go
 // straight into v_cvt_scalef32_pk_{fp8,bf8}_bf16 at scale 2^k (the code of
@@ -61,14 +59,11 @@
 #endif
 #ifndef ELY_SPLIT_CACHED_MB
 // split path: MB of x the |x|max launch reads last with plain loads instead
-// of nontemporal ones.  C4 per-tensor: quantize 0.408 -> 0.403 ms, round
-// trip 0.509 -> 0.499 ms (0, 192, 256 and 384 MB measured; a convert launch
+// of nontemporal ones.  C4 per-tensor, when measured: quantize 0.408 -> 0.403 ms, round
+// trip 0.509 -> 0.499 ms (0, 192, 256 and 384 MB; a convert launch
 // taking the segments last to first, to start on the cached ones, was
 // slower)
 #define ELY_SPLIT_CACHED_MB 256
-#endif
-#ifndef ELY_SPLIT_BATCH
-#define ELY_SPLIT_BATCH 1  // split path: vectors per lane per load batch of the convert launch (0: all)
 #endif
 #ifndef ELY_Q_LDS
 // wave-per-row quantize: unused dynamic LDS per block, capping it at 16
@@ -434,15 +429,31 @@ __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t value) {
 }
 
 // Long rows (and per-tensor scaling, one row) go through segments of
-// kSegElems elements.  The row's |x|max is reduced without atomics: wave
-// (r, j) of the rowmax_partial_kernel folds segments j, j + wpr, ... of row r
-// into partial[r * wpr + j]; rowmax_reduce_kernel folds a row's wpr partials
-// (wpr == 1: the partials are the row maxima).  Values are |x| bit patterns
-// (fp32 bits for fp32 input, bf16 bits for bf16), so max is an integer max.
+// kSegElems elements.  The row's |x|max is reduced without atomics: block
+// (r, j) of the rowmax_partial_kernel folds row r's segments, its waves'
+// maxima meeting in LDS, into partial[r * bpr + j], at most 256 a row; every
+// wave of the convert launch folds its row's partials itself while its segment
+// is on the way.  Per tensor, bf16, back to back, against a launch between
+// the two that folded up to 2,048 partials (and blocks of one wave): 0.4 M
+// elements 7.1 us against 10.3, 3.1 M 7.6 against 10.6, 16.8 M 12.8 against
+// 16.6, 33.6 M 25.4 against 28.5, 537 M 386 against 390; of a length that is
+// no whole number of vectors, 3.1 M 7.8 against 29.3.  Values are |x| bit
+// patterns (fp32 bits for fp32 input, bf16 bits for bf16), so max is an
+// integer max.
 constexpr int64_t kSplitWaves = ELY_SPLIT_WAVES;  // waves of the partial-max launch (at most)
+constexpr int kSplitBlockWaves = 8;               // ... per block, when a row has that many
 
-static int64_t split_wpr(int64_t rows, int64_t segs) {
-    return std::max<int64_t>(1, std::min<int64_t>(segs, kSplitWaves / std::max<int64_t>(rows, 1)));
+// How the partial-max launch shares a row: `waves` per block, `blocks` per row.
+struct SplitShape {
+    int waves;
+    int64_t blocks;
+};
+static SplitShape split_shape(int64_t rows, int64_t segs) {
+    const int64_t wpr = std::max<int64_t>(1, std::min<int64_t>(segs, kSplitWaves / std::max<int64_t>(rows, 1)));
+    if (wpr < kSplitBlockWaves) return {1, wpr};
+    // a multiple of the 8 XCDs for a single row (see rowmax_partial_kernel)
+    const int64_t blocks = (wpr + kSplitBlockWaves - 1) / kSplitBlockWaves;
+    return {kSplitBlockWaves, rows == 1 ? (blocks + 7) / 8 * 8 : blocks};
 }
 
 // Vectors of one segment a lane holds: 2048 bf16 = 256 x 16 B -> 4 per lane.
@@ -452,25 +463,51 @@ struct Seg {
     static constexpr int VPL = (int)(kSegElems / EPV / kWave);
 };
 
-// |x|max bits of elements [e0, e1) of row `row` (e1 - e0 <= kSegElems).
+// Segment `seg` of a row of cols elements (at least one vector of them): its
+// first element, whether it is a whole one, its vectors, and where vector vi
+// lies from e0.  A row that is no whole number of vectors ends in its last
+// EPV elements (row_vec_off), which may begin before the segment.
+template <bool BF16>
+struct SegAt {
+    static constexpr int EPV = Seg<BF16>::EPV, ESZ = BF16 ? 2 : 4;
+    int64_t e0;
+    bool whole;
+    int len, nv;
+    __device__ __forceinline__ SegAt(int64_t seg, int64_t cols)
+        : e0(seg * kSegElems), whole(e0 + kSegElems <= cols), len((int)min(kSegElems, cols - e0)),
+          nv((len + EPV - 1) / EPV) {}
+    __device__ __forceinline__ int off(int vi) const { return whole ? vi * EPV : min(vi * EPV, len - EPV); }
+};
+
+// That segment of the row at xr in registers; lanes past a short segment's
+// end load its last vector again.  Whole segments, nearly all of them, load
+// without the clamps (with them C4's |x|max pass took 184 us against 153).
+template <bool BF16, bool NT = (ELY_FP8_NT & 1) != 0>
+__device__ __forceinline__ void load_segment(const char* xr, const SegAt<BF16>& at, int lane,
+                                             uint4 (&buf)[Seg<BF16>::VPL]) {
+    const char* xs = xr + at.e0 * SegAt<BF16>::ESZ;
+    if (at.whole) {
+#pragma unroll
+        for (int j = 0; j < Seg<BF16>::VPL; ++j) buf[j] = ld_vec<NT>(xs + (lane + kWave * j) * 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < Seg<BF16>::VPL; ++j) buf[j] = ld_vec<NT>(xs + at.off(lane + kWave * j) * SegAt<BF16>::ESZ);
+    }
+}
+
+// |x|max bits of segment `seg` of row `row`; vec: the row holds at least one
+// vector.
 template <bool BF16, bool NT>
-__device__ __forceinline__ uint32_t seg_absmax(const void* x, int64_t row, int64_t cols, int64_t e0, int64_t e1,
-                                               int vec, int lane) {
-    constexpr int EPV = Seg<BF16>::EPV, VPL = Seg<BF16>::VPL, ESZ = BF16 ? 2 : 4;
+__device__ __forceinline__ uint32_t seg_absmax(const void* x, int64_t row, int64_t cols, int64_t seg, int vec, int lane) {
+    constexpr int VPL = Seg<BF16>::VPL, ESZ = BF16 ? 2 : 4;
     uint32_t amax = 0;
     if (vec) {
-        const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + (row * cols + e0) * ESZ);
-        const int64_t nv = (e1 - e0) / EPV;
         uint4 buf[VPL];
+        load_segment<BF16, NT>(static_cast<const char*>(x) + row * cols * ESZ, SegAt<BF16>(seg, cols), lane, buf);
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            const int64_t vi = lane + (int64_t)kWave * j;
-            buf[j] = ld_vec<NT>(xr + (vi < nv ? vi : nv - 1));
-        }
-#pragma unroll
-        for (int j = 0; j < VPL; ++j)
-            if (lane + (int64_t)kWave * j < nv) amax = vec_absmax<BF16>(buf[j], amax);
+        for (int j = 0; j < VPL; ++j) amax = vec_absmax<BF16>(buf[j], amax);
     } else {
+        const int64_t e0 = seg * kSegElems, e1 = min(e0 + kSegElems, cols);
         for (int64_t e = e0 + lane; e < e1; e += kWave) {
             uint32_t b = BF16 ? (uint32_t)static_cast<const uint16_t*>(x)[row * cols + e] & 0x7FFFu
                               : __float_as_uint(static_cast<const float*>(x)[row * cols + e]) & 0x7FFFFFFFu;
@@ -480,102 +517,112 @@ __device__ __forceinline__ uint32_t seg_absmax(const void* x, int64_t row, int64
     return amax;
 }
 
-template <bool BF16>
-__global__ __launch_bounds__(kQBlock) void rowmax_partial_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
-                                                                 int64_t segs, int64_t wpr, int vec, int64_t cached,
-                                                                 uint32_t* __restrict__ partial) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
-    if (gw >= rows * wpr) return;
-    const int64_t row = gw / wpr, j = gw % wpr;
+template <bool BF16, int W>
+__global__ __launch_bounds__(W * kWave) void rowmax_partial_kernel(const void* __restrict__ x, int64_t cols,
+                                                                   int64_t segs, int64_t bpr, int vec, int64_t cached,
+                                                                   uint32_t* __restrict__ partial) {
+    __shared__ uint32_t red[W];
+    const int lane = threadIdx.x & (kWave - 1), w = wave_uniform(threadIdx.x / kWave);
+    const int64_t row = blockIdx.x / bpr, j = blockIdx.x % bpr, step = bpr * W;
     uint32_t amax = 0;
     // a row's last `cached` segments are read last, with plain loads; two
     // loops in sequence keep the two kinds of loads apart
     const int64_t cut = segs - cached;
-    int64_t seg = j;
-    for (; seg < cut; seg += wpr) {
-        const int64_t e0 = seg * kSegElems;
-        amax = max(amax, seg_absmax<BF16, (ELY_FP8_NT & 1) != 0>(x, row, cols, e0, min(e0 + kSegElems, cols), vec, lane));
-    }
-    for (; seg < segs; seg += wpr) {
-        const int64_t e0 = seg * kSegElems;
-        amax = max(amax, seg_absmax<BF16, false>(x, row, cols, e0, min(e0 + kSegElems, cols), vec, lane));
-    }
+    // Block j's segments are j, j + bpr, ...: blocks go to the XCDs in turn,
+    // so with bpr a multiple of their number a single row's segment is read by
+    // the XCD that converts it, whose L2 may still hold it (32 M bf16: the
+    // convert launch 15.5 us, against 19 with segments 8 j, 8 j + 1, ...)
+    int64_t seg = j + w * bpr;
+    for (; seg < cut; seg += step) amax = max(amax, seg_absmax<BF16, (ELY_FP8_NT & 1) != 0>(x, row, cols, seg, vec, lane));
+    for (; seg < segs; seg += step) amax = max(amax, seg_absmax<BF16, false>(x, row, cols, seg, vec, lane));
     amax = wave_max_u32(amax);
-    if (lane == 0) partial[gw] = amax;
+    if (W == 1) {
+        if (lane == 0) partial[blockIdx.x] = amax;
+        return;
+    }
+    if (lane == 0) red[w] = amax;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int i = 1; i < W; ++i) amax = max(amax, red[i]);
+        partial[blockIdx.x] = amax;
+    }
 }
 
-__global__ __launch_bounds__(kRowBlock) void rowmax_reduce_kernel(const uint32_t* __restrict__ partial, int64_t rows,
-                                                                int64_t wpr, uint32_t* __restrict__ rowmax) {
-    __shared__ uint32_t red[kRowWaves];
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+// rowmax[r] = the max of row r's partials, one wave per row (the recovery's
+// launches read it).
+__global__ __launch_bounds__(kWave) void rowmax_reduce_kernel(const uint32_t* __restrict__ partial, int64_t rows,
+                                                              int64_t bpr, uint32_t* __restrict__ rowmax) {
     for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
         uint32_t m = 0;
-        for (int64_t i = threadIdx.x; i < wpr; i += kRowBlock) m = max(m, partial[r * wpr + i]);
+        for (int64_t i = threadIdx.x; i < bpr; i += kWave) m = max(m, partial[r * bpr + i]);
         m = wave_max_u32(m);
-        if (lane == 0) red[w] = m;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t t = red[0];
-            for (int k = 1; k < kRowWaves; ++k) t = max(t, red[k]);
-            rowmax[r] = t;
-        }
-        __syncthreads();
+        if (threadIdx.x == 0) rowmax[r] = m;
     }
 }
 
-// Segment `seg` of row `row` converted at the row's scale rs (the split
-// path's convert launch and the hint path's fixup).
+// Vector vi of a segment converted at the row's scale rs.
+template <int FMT, bool BF16>
+__device__ __forceinline__ void convert_seg_vec(const uint4& v, const SegAt<BF16>& at, int vi, int64_t base, const RowScale& rs,
+                                                uint8_t* q, void* out) {
+    if (vi >= at.nv) return;
+    const int64_t e = base + at.e0 + at.off(vi);
+    uint32_t words[2];
+    quant_vec_fast<FMT, BF16>(v, rs, words, out ? static_cast<char*>(out) + e * SegAt<BF16>::ESZ : nullptr);
+    if (q) {
+        if (BF16) st_vec2(q + e, make_uint2(words[0], words[1]));
+        else st_u32(q + e, words[0]);
+    }
+}
+
+// A segment converted at the row's scale rs, one vector per lane loaded and
+// stored at a time.
 template <int FMT, bool BF16>
 __device__ __forceinline__ void quant_segment(const void* x, int64_t row, int64_t cols, int64_t seg, int vec,
                                               const RowScale& rs, uint8_t* q, void* out, int lane) {
-    constexpr int EPV = Seg<BF16>::EPV, VPL = Seg<BF16>::VPL, ESZ = BF16 ? 2 : 4;
-    const int64_t e0 = seg * kSegElems, e1 = min(e0 + kSegElems, cols);
     const int64_t base = row * cols;
     if (vec && rs.fast) {
-        const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + (base + e0) * ESZ);
-        const int64_t nv = (e1 - e0) / EPV;
-        constexpr int SB = (ELY_SPLIT_BATCH <= 0 || ELY_SPLIT_BATCH > VPL) ? VPL : ELY_SPLIT_BATCH;
-        uint4 buf[VPL];
+        const SegAt<BF16> at(seg, cols);
+        const char* xs = static_cast<const char*>(x) + (base + at.e0) * SegAt<BF16>::ESZ;
 #pragma unroll
-        for (int j0 = 0; j0 < VPL; j0 += SB) {
-#pragma unroll
-            for (int j = j0; j < j0 + SB && j < VPL; ++j) {
-                const int64_t vi = lane + (int64_t)kWave * j;
-                buf[j] = ld_vec(xr + (vi < nv ? vi : nv - 1));
-            }
-#pragma unroll
-            for (int j = j0; j < j0 + SB && j < VPL; ++j) {
-                const int64_t vi = lane + (int64_t)kWave * j;
-                if (vi >= nv) continue;
-                uint32_t words[2];
-                const int64_t e = e0 + vi * EPV;
-                quant_vec_fast<FMT, BF16>(buf[j], rs, words, out ? static_cast<char*>(out) + (base + e) * ESZ : nullptr);
-                if (q) {
-                    if (BF16) st_vec2(q + base + e, make_uint2(words[0], words[1]));
-                    else st_u32(q + base + e, words[0]);
-                }
-            }
-            if (SB < VPL) __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < Seg<BF16>::VPL; ++j) {
+            const int vi = lane + kWave * j;
+            const uint4 v = ld_vec(xs + at.off(vi) * SegAt<BF16>::ESZ);
+            convert_seg_vec<FMT, BF16>(v, at, vi, base, rs, q, out);
+            __builtin_amdgcn_sched_barrier(0);
         }
     } else {
-        quant_slow<FMT, BF16>(x, base, e0, e1, rs, q, out, lane);
+        quant_slow<FMT, BF16>(x, base, seg * kSegElems, min((seg + 1) * kSegElems, cols), rs, q, out, lane);
     }
 }
 
 template <int FMT, bool BF16>
 __global__ __launch_bounds__(kQBlock) void quant_split_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
                                                               int64_t segs, int vec,
-                                                              const uint32_t* __restrict__ rowmax,
+                                                              const uint32_t* __restrict__ partial, int64_t bpr,
                                                               uint8_t* __restrict__ q, int32_t* __restrict__ k,
                                                               void* __restrict__ out) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     const int64_t row = gw / segs, seg = gw % segs;
     if (row >= rows) return;
-    const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(rowmax[row]), BF16, BF16);
+    // the segment is on its way while the row's partials are folded
+    const SegAt<BF16> at(seg, cols);
+    uint4 buf[Seg<BF16>::VPL];
+    if (vec) load_segment<BF16>(static_cast<const char*>(x) + row * cols * SegAt<BF16>::ESZ, at, lane, buf);
+    uint32_t m = 0;
+#pragma unroll 4
+    for (int64_t i = lane; i < bpr; i += kWave) m = max(m, partial[row * bpr + i]);
+    m = wave_max_u32(m);
+    const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(m), BF16, BF16);
     if (seg == 0 && lane == 0 && k) k[row] = rs.k;
-    quant_segment<FMT, BF16>(x, row, cols, seg, vec, rs, q, out, lane);
+    if (vec && rs.fast) {
+#pragma unroll
+        for (int j = 0; j < Seg<BF16>::VPL; ++j)
+            convert_seg_vec<FMT, BF16>(buf[j], at, lane + kWave * j, row * cols, rs, q, out);
+    } else {
+        quant_slow<FMT, BF16>(x, row * cols, at.e0, at.e0 + at.len, rs, q, out, lane);
+    }
 }
 
 // ------------------------------------------------- per-tensor, with a hint
@@ -623,7 +670,7 @@ __global__ __launch_bounds__(kQBlock) void quant_hint_kernel(const void* __restr
                                                              int32_t hint_is_amax, uint8_t* __restrict__ q,
                                                              void* __restrict__ out, uint32_t* __restrict__ partial,
                                                              int32_t* __restrict__ hint_copy) {
-    constexpr int EPV = Seg<BF16>::EPV, VPL = Seg<BF16>::VPL, ESZ = BF16 ? 2 : 4;
+    constexpr int VPL = Seg<BF16>::VPL;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t seg = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     if (seg >= segs) return;
@@ -639,29 +686,14 @@ __global__ __launch_bounds__(kQBlock) void quant_hint_kernel(const void* __restr
     hs.fast = true;
     hs.s_down = __uint_as_float((uint32_t)(127 - hint) << 23);
     hs.s_up = __uint_as_float((uint32_t)(127 + hint) << 23);
-    const int64_t e0 = seg * kSegElems;
-    const int64_t nv = (min(e0 + kSegElems, n) - e0) / EPV;
-    const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + e0 * ESZ);
     uint4 buf[VPL];
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        const int64_t vi = lane + (int64_t)kWave * j;
-        buf[j] = ld_vec(xr + (vi < nv ? vi : nv - 1));
-    }
+    const SegAt<BF16> at(seg, n);
+    load_segment<BF16>(static_cast<const char*>(x), at, lane, buf);
     uint32_t amax = 0;
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
-        const int64_t vi = lane + (int64_t)kWave * j;
-        if (vi >= nv) continue;
         amax = vec_absmax<BF16>(buf[j], amax);
-        if (!convert) continue;
-        uint32_t words[2];
-        const int64_t e = e0 + vi * EPV;
-        quant_vec_fast<FMT, BF16>(buf[j], hs, words, out ? static_cast<char*>(out) + e * ESZ : nullptr);
-        if (q) {
-            if (BF16) st_vec2(q + e, make_uint2(words[0], words[1]));
-            else st_u32(q + e, words[0]);
-        }
+        if (convert) convert_seg_vec<FMT, BF16>(buf[j], at, lane + kWave * j, 0, hs, q, out);
     }
     amax = wave_max_u32(amax);
     if (lane == 0) partial[seg] = amax;
@@ -675,24 +707,10 @@ __global__ __launch_bounds__(kQBlock) void quant_hint_kernel(const void* __restr
 template <bool BF16>
 __global__ __launch_bounds__(kQBlock) void guess_amax_kernel(const void* __restrict__ x, int64_t n, int64_t stride,
                                                              int64_t samples, uint32_t* __restrict__ partial) {
-    constexpr int EPV = Seg<BF16>::EPV, VPL = Seg<BF16>::VPL, ESZ = BF16 ? 2 : 4;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t w = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     if (w >= samples) return;
-    const int64_t e0 = w * stride * kSegElems;
-    const int64_t nv = (min(e0 + kSegElems, n) - e0) / EPV;
-    const uint4* xr = reinterpret_cast<const uint4*>(static_cast<const char*>(x) + e0 * ESZ);
-    uint4 buf[VPL];
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        const int64_t vi = lane + (int64_t)kWave * j;
-        buf[j] = ld_vec(xr + (vi < nv ? vi : nv - 1));
-    }
-    uint32_t m = 0;
-#pragma unroll
-    for (int j = 0; j < VPL; ++j)
-        if (lane + (int64_t)kWave * j < nv) m = vec_absmax<BF16>(buf[j], m);
-    m = wave_max_u32(m);
+    const uint32_t m = wave_max_u32(seg_absmax<BF16, (ELY_FP8_NT & 1) != 0>(x, 0, n, w * stride, 1, lane));
     if (lane == 0) partial[w] = to_f32_bits<BF16>(m);
 }
 
@@ -1423,13 +1441,18 @@ static bool whole_vecs(int64_t cols, int32_t dtype, const void* x, const uint8_t
            (!q || reinterpret_cast<uintptr_t>(q) % (uintptr_t)epv == 0);
 }
 
-// A row's vectors in units of one per lane of a wave (kWave vectors), for any
-// row of at least one vector at any element's alignment that the register
-// paths take; 0 for the others.
-static int rows_units(int64_t cols, int32_t dtype, const void* x, const void* out) {
+// Whether these rows take the vector paths: at least one vector, at any
+// element's alignment.
+static bool any_vecs(int64_t cols, int32_t dtype, const void* x, const void* out) {
     const int64_t epv = dtype == ELY_BF16 ? 8 : 4, esz = dtype == ELY_BF16 ? 2 : 4;
-    if (cols < epv || reinterpret_cast<uintptr_t>(x) % esz || reinterpret_cast<uintptr_t>(out) % esz) return 0;
-    const int64_t per = epv * kWave;
+    return cols >= epv && reinterpret_cast<uintptr_t>(x) % esz == 0 && reinterpret_cast<uintptr_t>(out) % esz == 0;
+}
+
+// A row's vectors in units of one per lane of a wave (kWave vectors), for
+// rows that the register paths take; 0 for the others.
+static int rows_units(int64_t cols, int32_t dtype, const void* x, const void* out) {
+    const int64_t per = (dtype == ELY_BF16 ? 8 : 4) * kWave;
+    if (!any_vecs(cols, dtype, x, out)) return 0;
     return cols <= per * kMaxRowUnits ? (int)((cols + per - 1) / per) : 0;
 }
 
@@ -1458,22 +1481,39 @@ static size_t split_ws_bytes(int64_t rows) {
     return rowmax_bytes(rows) + align_up((size_t)std::max<int64_t>(rows, kSplitWaves) * 4, 256);
 }
 
-// rowmax[r] = |x|max bits of row r, through the split path's two launches.
+// partial[r * shape.blocks + j]: the partial |x|max bits of row r, from the
+// split path's first launch.
+template <bool BF16>
+static SplitShape split_partials(const void* x, int64_t rows, int64_t cols, int vec, uint32_t* partial, hipStream_t s) {
+    const int64_t segs = (cols + kSegElems - 1) / kSegElems;
+    const SplitShape sh = split_shape(rows, segs);
+    if (rows > INT64_MAX / (sh.blocks * sh.waves)) fail(ELY_EINVAL, "too many rows");
+    const int64_t blocks = rows * sh.blocks;
+    // a dispatch counts its work-items in 32 bits
+    if (blocks > 0xFFFFFFFFLL / (sh.waves * kWave)) fail(ELY_EINVAL, "grid too large: more than 2^32 - 1 threads in one launch");
+    const int64_t seg_bytes = kSegElems * (BF16 ? 2 : 4);
+    const int64_t cached = std::min<int64_t>(segs, ((int64_t)ELY_SPLIT_CACHED_MB << 20) / (seg_bytes * rows));
+    if (sh.waves == 1)
+        hipLaunchKernelGGL((rowmax_partial_kernel<BF16, 1>), dim3((unsigned)blocks), dim3(kWave), 0, s, x, cols, segs,
+                           sh.blocks, vec, cached, partial);
+    else
+        hipLaunchKernelGGL((rowmax_partial_kernel<BF16, kSplitBlockWaves>), dim3((unsigned)blocks),
+                           dim3(kSplitBlockWaves * kWave), 0, s, x, cols, segs, sh.blocks, vec, cached, partial);
+    check_launch("rowmax_partial_kernel");
+    return sh;
+}
+
+// rowmax[r] = |x|max bits of row r, through the split path's first launch and
+// a fold of its partials.
 template <bool BF16>
 static void split_rowmax(const void* x, int64_t rows, int64_t cols, int vec, void* workspace, uint32_t* rowmax,
                          hipStream_t s) {
-    const int64_t segs = (cols + kSegElems - 1) / kSegElems;
-    const int64_t wpr = split_wpr(rows, segs);
-    if (rows > INT64_MAX / wpr) fail(ELY_EINVAL, "too many rows");
-    uint32_t* partial = wpr == 1 ? rowmax : reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + rowmax_bytes(rows));
-    const int64_t seg_bytes = kSegElems * (BF16 ? 2 : 4);
-    const int64_t cached = std::min<int64_t>(segs, ((int64_t)ELY_SPLIT_CACHED_MB << 20) / (seg_bytes * rows));
-    hipLaunchKernelGGL((rowmax_partial_kernel<BF16>), dim3(blocks_for_waves(rows * wpr)), dim3(kQBlock), 0, s, x, rows,
-                       cols, segs, wpr, vec, cached, partial);
-    check_launch("rowmax_partial_kernel");
-    if (wpr > 1) {
-        hipLaunchKernelGGL(rowmax_reduce_kernel, dim3((unsigned)std::min<int64_t>(rows, 65536)), dim3(kRowBlock), 0, s,
-                           (const uint32_t*)partial, rows, wpr, rowmax);
+    const bool one = split_shape(rows, (cols + kSegElems - 1) / kSegElems).blocks == 1;
+    uint32_t* partial = one ? rowmax : reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + rowmax_bytes(rows));
+    const SplitShape sh = split_partials<BF16>(x, rows, cols, vec, partial, s);
+    if (!one) {
+        hipLaunchKernelGGL(rowmax_reduce_kernel, dim3((unsigned)std::min<int64_t>(rows, 65536)), dim3(kWave), 0, s,
+                           (const uint32_t*)partial, rows, sh.blocks, rowmax);
         check_launch("rowmax_reduce_kernel");
     }
 }
@@ -1497,7 +1537,7 @@ static void quantize_impl(const void* x, int64_t rows, int64_t cols, uint8_t* q,
         return;
     }
     const int32_t dt = BF16 ? ELY_BF16 : ELY_F32;
-    const int vec = whole_vecs(cols, dt, x, q, out);
+    const int vec = any_vecs(cols, dt, x, out);
     const bool want_ws = wants_workspace(cols, dt, x, q, out);
     const bool guess = want_ws && allow_guess && rows == 1 && (q || out) && vec &&
                        cols >= ((int64_t)ELY_GUESS_MIN_MB << 20) / (BF16 ? 2 : 4) && workspace &&
@@ -1520,13 +1560,13 @@ static void quantize_impl(const void* x, int64_t rows, int64_t cols, uint8_t* q,
         return dispatch_rows<FMT, BF16>(units, x, rows, cols, q, k, out, s);
     }
     if (guess) return quantize_guess_impl<FMT, BF16>(x, cols, q, k, out, workspace, ws_bytes, s);
-    uint32_t* rowmax = static_cast<uint32_t*>(workspace);
+    uint32_t* partial = static_cast<uint32_t*>(workspace);
     const int64_t segs = (cols + kSegElems - 1) / kSegElems;
     if (rows > INT64_MAX / segs) fail(ELY_EINVAL, "too many segments");
-    split_rowmax<BF16>(x, rows, cols, vec, workspace, rowmax, s);
     const unsigned blocks = blocks_for_waves(rows * segs);
+    const SplitShape sh = split_partials<BF16>(x, rows, cols, vec, partial, s);
     hipLaunchKernelGGL((quant_split_kernel<FMT, BF16>), dim3(blocks), dim3(kQBlock), 0, s, x, rows, cols, segs, vec,
-                       (const uint32_t*)rowmax, q, k, out);
+                       (const uint32_t*)partial, sh.blocks, q, k, out);
     check_launch("quant_split_kernel");
 }
 
@@ -1545,7 +1585,10 @@ static void quantize_hint_impl(const void* x, int64_t n, int32_t k_hint, const i
     if (!workspace || ws_bytes < (int64_t)hint_ws_bytes(n))
         fail(ELY_EWORKSPACE, "ely_fp8_quantize_hint: workspace of " + std::to_string(ws_bytes) + " bytes, need " +
                                  std::to_string(hint_ws_bytes(n)) + " (ely_fp8_hint_workspace_bytes)");
-    const bool vec = n > 0 && whole_vecs(n, BF16 ? ELY_BF16 : ELY_F32, x, q, out);
+    // a caller's hint keeps to whole aligned vectors (*hit says so); a guess
+    // takes any row of at least one
+    const int32_t dt = BF16 ? ELY_BF16 : ELY_F32;
+    const bool vec = n > 0 && (hint_is_amax ? any_vecs(n, dt, x, out) : whole_vecs(n, dt, x, q, out));
     if (!vec || (!k_hint_dev && (k_hint < -kFastK || k_hint > kFastK))) {
         // no one-pass form for this tensor or hint: the split path, a miss
         quantize_impl<FMT, BF16>(x, 1, n, q, k, out, workspace, ws_bytes, s, false);

@@ -148,8 +148,7 @@ int64_t ely_fp8_workspace_bytes(int64_t rows, int64_t cols, int32_t x_dtype);
  * rows = 1.  x: [rows, cols] bf16 or fp32; q: [rows, cols] bytes, or NULL to
  * compute k alone (fp8.scale_exp); k: [rows] int32.
  * A row that fits no register path is read twice (its |x|max, then its
- * codes), except one row of at least 64 MiB (16-byte aligned, whole
- * vectors) given the larger workspace: its exponent is guessed from every
+ * codes), except one row of at least 64 MiB given the larger workspace: its exponent is guessed from every
  * 61st 2,048-element segment and the codes are made at the guess in the
  * same pass that finds |x|max (as ely_fp8_quantize_hint does), a second
  * pass following only when the guess was wrong.  The bytes are the same

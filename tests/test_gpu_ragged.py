@@ -73,3 +73,37 @@ def test_ragged_dequantize_with_a_distinct_exponent_per_row(oracle, fmt, cols):
             d = bits(fp8.dequantize(q, k, DT[out])).reshape(-1)
             od = oracle.dequantize(codes.reshape(rows, cols), kk, fmt, out).reshape(-1)
             assert f32_equal(d, od) if out == "f32" else np.array_equal(d, od)
+
+
+# per tensor around a vector, a segment (2,048 elements), one block's and every
+# block's share of the |x|max launch, and past the sampled guess's 64 MiB
+@pytest.mark.parametrize("dname", ["bf16", "f32"])
+@pytest.mark.parametrize("n", [32777, 40 * 2048 + 1, 64 * 2048 - 3, 2048 * 2048 + 2047, 2049 * 2048 + 6])
+def test_per_tensor_of_any_length_equals_the_oracle(oracle, dname, n):
+    base = activation((n + 1,), seed=n % 97, dtype=DT[dname])
+    for off in (0, 1):
+        x = base[off : off + n]
+        say("fp8 ragged per tensor", dname, n, "offset", off)
+        _codec_equals_the_oracle(oracle, x.reshape(1, n), "e4m3" if off else "e5m2")
+
+
+@pytest.mark.parametrize("off", [0, 3])
+def test_a_ragged_tensor_past_the_guess_size_equals_torch(off):
+    """An odd length of over 64 MiB, its largest value in the vector that
+    overlaps the last whole segment, against torch's own ops on this GPU."""
+    from elysium_wan_amd import fp8
+
+    n = (1 << 25) + 2048 + 5
+    g = torch.Generator(device="cuda").manual_seed(off)
+    x = torch.randn(n + off, generator=g, device="cuda").bfloat16()[off:]
+    for top in (None, 1e4):
+        if top is not None:
+            x[n - 2] = top
+        say("fp8 ragged guess", off, top)
+        q, k = fp8.quantize(x, "e4m3", per_tensor=True)
+        amax = x.abs().max().float()
+        kref = int(torch.frexp(amax).exponent) - 8
+        assert int(k) == kref
+        qref = (x * 2.0**-kref).to(torch.float8_e4m3fn)
+        assert torch.equal(q.view(torch.uint8), qref.view(torch.uint8))
+        assert torch.equal(fp8.roundtrip(x, "e4m3", per_tensor=True), qref.to(torch.bfloat16) * 2.0**kref)
