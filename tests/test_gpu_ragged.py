@@ -107,3 +107,24 @@ def test_a_ragged_tensor_past_the_guess_size_equals_torch(off):
         qref = (x * 2.0**-kref).to(torch.float8_e4m3fn)
         assert torch.equal(q.view(torch.uint8), qref.view(torch.uint8))
         assert torch.equal(fp8.roundtrip(x, "e4m3", per_tensor=True), qref.to(torch.bfloat16) * 2.0**kref)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 257, 4099])
+def test_cast_fold_and_widen_at_any_address(n):
+    """Views off the 16-byte (fp32) and 8-byte (bf16) boundary against torch's
+    own cast and adds, and nothing written beside them."""
+    from elysium_wan_amd import pieces
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for off in (0, 1, 2, 3):
+        say("pieces at any address", n, off)
+        x = torch.randn(n + 8, generator=g, device="cuda")
+        h = torch.randn(n + 8, generator=g, device="cuda").bfloat16()
+        assert torch.equal(pieces.cast_piece(x[off : off + n], torch.bfloat16), x[off : off + n].bfloat16())
+        assert torch.equal(pieces.fold_start(h[off : off + n]), h[off : off + n].float())
+        for acc, part in ((x, h), (x, x.flip(0)), (h, x), (h, h.flip(0))):
+            got, want = acc.clone(), acc.clone()
+            # torch's in-place add into bf16 is the fp32 sum rounded once
+            want[off : off + n] = (acc[off : off + n].float() + part[1 : n + 1].float()).to(acc.dtype)
+            pieces.fold_add(got[off : off + n], part[1 : n + 1])
+            assert torch.equal(got, want)
