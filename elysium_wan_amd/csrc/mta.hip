@@ -141,7 +141,7 @@ struct NormDesc {          // 40 bytes
     int64_t numel;
     int64_t tile_begin;
     int32_t dtype;         // ELY_F32 | ELY_BF16
-    int32_t aligned;       // g (and acc) 16-byte aligned
+    int32_t vec;           // g (and acc) at an element's address: moved as vectors
 };
 
 // Sum of squares of 8 values by a fixed fp32 tree.
@@ -164,13 +164,27 @@ __device__ __forceinline__ const ELY_GLOBAL T* gp(const T* p) {
     return (const ELY_GLOBAL T*)p;
 }
 
-typedef float nf32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t nu32x4 __attribute__((ext_vector_type(4)));
+// The same at any element's address: gfx950 moves a vector off its 16-byte
+// boundary with the same instruction, so tensors packed back to back take
+// the vector paths too.  41 M elements packed at an odd width, against the
+// element paths: clip_grad_norm_ 397 -> 239 us (fp32) and 308 -> 136 (bf16),
+// the clipped step 981 -> 727 (bf16 gradients) and 998 -> 808 (fp32).
+typedef uint32_t nu32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 
-template <typename T, bool NT = ELY_NORM_NT != 0>
-__device__ __forceinline__ T ld_norm(const ELY_GLOBAL T* p) {
-    if (NT) return __builtin_nontemporal_load(p);
-    return *p;
+// Whether p is at an element's address.
+static bool elem_aligned(const void* p, int32_t dtype) {
+    return reinterpret_cast<uintptr_t>(p) % (dtype == ELY_BF16 ? 2 : 4) == 0;
+}
+
+template <bool NT = ELY_NORM_NT != 0>
+__device__ __forceinline__ nu32x4 ld_norm(const void* p) {
+    const ELY_GLOBAL nu32x4_u* v = (const ELY_GLOBAL nu32x4_u*)p;
+    if (NT) return __builtin_nontemporal_load(v);
+    return *v;
+}
+__device__ __forceinline__ void st_norm(void* p, nu32x4 v) {
+    __builtin_nontemporal_store((nu32x4_u)v, (ELY_GLOBAL nu32x4_u*)p);
 }
 
 // The raw 16-byte vectors of one 8-element group: 1 (bf16) or 2 (fp32)
@@ -178,18 +192,17 @@ __device__ __forceinline__ T ld_norm(const ELY_GLOBAL T* p) {
 template <bool BF16, bool FOLD>
 struct Raw8 {
     nu32x4 g[BF16 ? 1 : 2];
-    nf32x4 a[FOLD ? 2 : 1];
+    nu32x4 a[FOLD ? 2 : 1];
 };
 
 template <bool BF16, bool FOLD, bool NT>
 __device__ __forceinline__ void raw8_load(const NormDesc& d, int64_t i, Raw8<BF16, FOLD>& r) {
-    const ELY_GLOBAL nu32x4* p = gp(reinterpret_cast<const nu32x4*>(static_cast<const char*>(d.g) + i * (BF16 ? 2 : 4)));
-    r.g[0] = ld_norm<nu32x4, NT>(p);
-    if (!BF16) r.g[BF16 ? 0 : 1] = ld_norm<nu32x4, NT>(p + 1);
+    const char* p = static_cast<const char*>(d.g) + i * (BF16 ? 2 : 4);
+    r.g[0] = ld_norm<NT>(p);
+    if (!BF16) r.g[BF16 ? 0 : 1] = ld_norm<NT>(p + 16);
     if (FOLD) {
-        const ELY_GLOBAL nf32x4* q = gp(reinterpret_cast<const nf32x4*>(d.acc + i));
-        r.a[0] = ld_norm<nf32x4, NT>(q);
-        r.a[FOLD ? 1 : 0] = ld_norm<nf32x4, NT>(q + 1);
+        r.a[0] = ld_norm<NT>(d.acc + i);
+        r.a[FOLD ? 1 : 0] = ld_norm<NT>(d.acc + i + 4);
     }
 }
 
@@ -213,14 +226,14 @@ __device__ __forceinline__ float raw8_sumsq(const Raw8<BF16, FOLD>& r) {
     if (FOLD) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            x[j] = r.a[0][j] + x[j];
-            x[4 + j] = r.a[FOLD ? 1 : 0][j] + x[4 + j];
+            x[j] = __uint_as_float(r.a[0][j]) + x[j];
+            x[4 + j] = __uint_as_float(r.a[FOLD ? 1 : 0][j]) + x[4 + j];
         }
     }
     return sq8(x);
 }
 
-// Sum of squares of one full, aligned tile: lane l owns the 8-element groups
+// Sum of squares of one full tile: lane l owns the 8-element groups
 // j*64 + l, j = 0..TILE/512-1, added in order; kNormUnroll groups' raw vectors are
 // loaded before the first of them is summed.
 template <bool BF16, bool FOLD, int64_t TILE, bool NT>
@@ -255,6 +268,26 @@ __device__ __forceinline__ void load8_any(const NormDesc& d, int64_t i, int64_t 
     }
 }
 
+// A tensor's last, short tile [e0, e1): the same groups in the same order,
+// whole ones as vectors, the one that crosses e1 element by element; groups
+// past it would add +0.0.
+template <bool BF16, bool FOLD, bool NT>
+__device__ __forceinline__ double part_sumsq(const NormDesc& d, int64_t e0, int64_t e1, int lane) {
+    double acc = 0.0;
+    for (int64_t i = e0 + lane * 8; i < e1; i += kWave * 8) {
+        if (i + 8 <= e1) {
+            Raw8<BF16, FOLD> r;
+            raw8_load<BF16, FOLD, NT>(d, i, r);
+            acc += (double)raw8_sumsq<BF16, FOLD>(r);
+        } else {
+            float x[8];
+            load8_any<FOLD>(d, i, e1, x);
+            acc += (double)sq8(x);
+        }
+    }
+    return acc;
+}
+
 // DT: the gradients' dtype when one call's are all ELY_F32 or all ELY_BF16
 // (the tile loop is then compiled for that dtype only, which keeps the
 // kernel's registers, and so its occupancy, to what that dtype needs), or -1
@@ -280,10 +313,14 @@ __device__ __forceinline__ void norm_tiles(const Desc* desc, int32_t n, int64_t&
         const int64_t e0 = (tile - d.tile_begin) * TILE;
         const int64_t e1 = min(e0 + TILE, d.numel);
         double acc = 0.0;
-        // lane l owns groups j*64 + l of 8 elements, in the same order on both paths
-        if (d.aligned && e1 - e0 == TILE) {
-            if (DT == ELY_BF16 || (DT < 0 && d.dtype == ELY_BF16)) acc = tile_sumsq_vec<true, FOLD, TILE, NT>(d, e0, lane);
+        // lane l owns groups j*64 + l of 8 elements, in the same order on every path
+        const bool bf16 = DT == ELY_BF16 || (DT < 0 && d.dtype == ELY_BF16);
+        if (d.vec && e1 - e0 == TILE) {
+            if (bf16) acc = tile_sumsq_vec<true, FOLD, TILE, NT>(d, e0, lane);
             else acc = tile_sumsq_vec<false, FOLD, TILE, NT>(d, e0, lane);
+        } else if (d.vec) {
+            if (bf16) acc = part_sumsq<true, FOLD, NT>(d, e0, e1, lane);
+            else acc = part_sumsq<false, FOLD, NT>(d, e0, e1, lane);
         } else {
             for (int j = 0; j < (int)(TILE / (kWave * 8)); ++j) {
                 float x[8];
@@ -380,11 +417,26 @@ __global__ __launch_bounds__(kFinalThreads) void norm_final_kernel(const double*
 #define ELY_CLIP_UNROLL 2    // clip scale: 16-byte vectors a lane loads before storing
 #endif
 
+// One 16-byte vector of 8 bf16 or 4 fp32 elements times coef, each product
+// rounded once to the dtype.
+__device__ __forceinline__ nu32x4 scale_vec(nu32x4 r, float coef, bool bf16) {
+    nu32x4 o;
+    if (bf16) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            o[k] = f32_to_bf16(bf16_to_f32(r[k] & 0xFFFFu) * coef) | (f32_to_bf16(bf16_to_f32(r[k] >> 16) * coef) << 16);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = __float_as_uint(__uint_as_float(r[k]) * coef);
+    }
+    return o;
+}
+
 // g <- g * coef in place, rounded once to g's dtype (torch's
 // _foreach_mul_(grads, clip_coef), clip_grad.py:170-177), over the norm's
-// own tile table: wave w scales tiles w, w + W, ...  A full, aligned tile
-// moves 16-byte vectors, lane l taking vectors l, l + 64, ...; others go
-// element by element.  DT as norm_partials_kernel.
+// own tile table: wave w scales tiles w, w + W, ...  A tile moves as 16-byte
+// vectors, lane l taking vectors l, l + 64, ...; what is left of a short tile
+// goes element by element.  DT as norm_partials_kernel.
 template <int DT, int64_t TILE, class Desc>
 __device__ __forceinline__ void clip_scale_body(const Desc* desc, int32_t n, int64_t total_tiles, const float* coef_ptr) {
     constexpr int U = ELY_CLIP_UNROLL;
@@ -400,34 +452,31 @@ __device__ __forceinline__ void clip_scale_body(const Desc* desc, int32_t n, int
         const bool bf16 = DT == ELY_BF16 || (DT < 0 && d.dtype == ELY_BF16);
         const int64_t e0 = (tile - d.tile_begin) * TILE;
         const int64_t e1 = min(e0 + TILE, d.numel);
-        if (d.aligned && e1 - e0 == TILE) {
-            nu32x4* base = reinterpret_cast<nu32x4*>(static_cast<char*>(const_cast<void*>(d.g)) + e0 * (bf16 ? 2 : 4));
-            const int nvec = (int)(TILE * (bf16 ? 2 : 4) / 16);
-            for (int j0 = 0; j0 < nvec; j0 += kWave * U) {
-                nu32x4 r[U];
+        int64_t done = e0;  // elements moved as vectors
+        if (d.vec) {
+            const int esz = bf16 ? 2 : 4;
+            char* base = static_cast<char*>(const_cast<void*>(d.g)) + e0 * esz;
+            if (e1 - e0 == TILE) {
+                const int nvec = (int)(TILE * esz / 16);
+                for (int j0 = 0; j0 < nvec; j0 += kWave * U) {
+                    nu32x4 r[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) r[u] = ld_norm(gp(base + j0 + u * kWave + lane));
+                    for (int u = 0; u < U; ++u) r[u] = ld_norm(base + (j0 + u * kWave + lane) * 16);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    nu32x4 o;
-                    if (bf16) {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            o[k] = f32_to_bf16(bf16_to_f32(r[u][k] & 0xFFFFu) * coef) |
-                                   (f32_to_bf16(bf16_to_f32(r[u][k] >> 16) * coef) << 16);
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) o[k] = __float_as_uint(__uint_as_float(r[u][k]) * coef);
-                    }
-                    __builtin_nontemporal_store(o, gp(base + j0 + u * kWave + lane));
+                    for (int u = 0; u < U; ++u) st_norm(base + (j0 + u * kWave + lane) * 16, scale_vec(r[u], coef, bf16));
                 }
+                continue;
             }
-        } else if (bf16) {
+            const int nvec = (int)((e1 - e0) * esz / 16);
+            for (int j = lane; j < nvec; j += kWave) st_norm(base + j * 16, scale_vec(ld_norm(base + j * 16), coef, bf16));
+            done = e0 + (int64_t)nvec * (16 / esz);
+        }
+        if (bf16) {
             uint16_t* g = static_cast<uint16_t*>(const_cast<void*>(d.g));
-            for (int64_t e = e0 + lane; e < e1; e += kWave) g[e] = (uint16_t)f32_to_bf16(bf16_to_f32(g[e]) * coef);
+            for (int64_t e = done + lane; e < e1; e += kWave) g[e] = (uint16_t)f32_to_bf16(bf16_to_f32(g[e]) * coef);
         } else {
             float* g = static_cast<float*>(const_cast<void*>(d.g));
-            for (int64_t e = e0 + lane; e < e1; e += kWave) g[e] = g[e] * coef;
+            for (int64_t e = done + lane; e < e1; e += kWave) g[e] = g[e] * coef;
         }
     }
 }
@@ -499,7 +548,7 @@ struct AdamDesc {          // 64 bytes
     uint16_t* copy;        // bf16 working copy or null
     int64_t numel;
     int32_t tile_begin;    // the launch checks that its tiles fit int32
-    int32_t aligned;       // every pointer 16-byte aligned
+    int32_t vec;           // every pointer at an element's address: moved as quads
 };
 static_assert(sizeof(AdamDesc) == 64, "AdamDesc is 64 bytes");
 
@@ -574,69 +623,71 @@ __device__ __forceinline__ i32x4 bits4(const float (&x)[4]) {
     return i32x4{__float_as_int(x[0]), __float_as_int(x[1]), __float_as_int(x[2]), __float_as_int(x[3])};
 }
 
-// Whole block steps of elements [e0, e0 + steps * kStep) of an aligned tensor.
+// The buffer resources of a range of one tensor's streams: `ne` elements from
+// element e0 on.
+template <bool BF16G, bool FOLD>
+struct AdamStreams {
+    __amdgpu_buffer_rsrc_t rp, rm, rv, rg, ra, rc;
+    __device__ __forceinline__ AdamStreams(const AdamDesc& d, int64_t e0, int32_t ne)
+        : rp(buf_rsrc(d.p + e0, ne * 4)), rm(buf_rsrc(d.m + e0, ne * 4)), rv(buf_rsrc(d.v + e0, ne * 4)),
+          rg(BF16G ? buf_rsrc(static_cast<const uint16_t*>(d.g) + e0, ne * 2)
+                   : buf_rsrc(static_cast<const float*>(d.g) + e0, ne * 4)),
+          ra(FOLD ? buf_rsrc(d.acc + e0, ne * 4) : rp), rc(d.copy ? buf_rsrc(d.copy + e0, ne * 2) : rp) {}
+};
+
+// The quad of elements [o, o + 4) of those streams.
 template <bool BF16G, int ORDER, bool WD, bool CLIP, bool FOLD>
-__device__ __forceinline__ void adam_steps(const AdamDesc& d, const ely_adamw_consts& c, float coef, int64_t e0,
-                                           int64_t steps) {
+__device__ __forceinline__ void adam_quad(const AdamStreams<BF16G, FOLD>& s, bool has_copy, const ely_adamw_consts& c,
+                                          float coef, int32_t o) {
     using Op = AdamOp<BF16G, ORDER, WD, CLIP, FOLD>;
-    const int32_t ne = (int32_t)(steps * kStep);  // a tile's range: at most kAdamTile elements
-    const __amdgpu_buffer_rsrc_t rp = buf_rsrc(d.p + e0, ne * 4), rm = buf_rsrc(d.m + e0, ne * 4),
-                                 rv = buf_rsrc(d.v + e0, ne * 4);
-    const __amdgpu_buffer_rsrc_t rg = BF16G ? buf_rsrc(static_cast<const uint16_t*>(d.g) + e0, ne * 2)
-                                            : buf_rsrc(static_cast<const float*>(d.g) + e0, ne * 4);
-    const __amdgpu_buffer_rsrc_t ra = FOLD ? buf_rsrc(d.acc + e0, ne * 4) : rp;
-    const __amdgpu_buffer_rsrc_t rc = d.copy ? buf_rsrc(d.copy + e0, ne * 2) : rp;
-    for (int64_t s = 0; s < steps; ++s) {
-        const int32_t o = (int32_t)(s * kStep) + (int32_t)threadIdx.x * 4;  // the lane's first element
-        // g (and the fold's accumulator), m and v are loaded ahead of p: the
-        // moments need only those, and m and v are stored before the sqrt
-        // and the division that p waits for (C1, alternating fresh
-        // processes, against loading p first and storing p, m, v after both
-        // halves: faster in 8 of 8 pairs in two sessions, 0.4-0.6 %, and
-        // even in a third)
-        i32x2 gw = {0, 0};
-        i32x4 ga = {0, 0, 0, 0}, A = {0, 0, 0, 0};
-        if (BF16G) gw = __builtin_amdgcn_raw_buffer_load_b64(rg, o * 2, 0, kBufNT);
-        else ga = __builtin_amdgcn_raw_buffer_load_b128(rg, o * 4, 0, kBufNT);
-        if (FOLD) A = __builtin_amdgcn_raw_buffer_load_b128(ra, o * 4, 0, kBufNT);
-        const i32x4 M = __builtin_amdgcn_raw_buffer_load_b128(rm, o * 4, 0, kBufNT);
-        const i32x4 V = __builtin_amdgcn_raw_buffer_load_b128(rv, o * 4, 0, kBufNT);
-        const i32x4 P = __builtin_amdgcn_raw_buffer_load_b128(rp, o * 4, 0, kBufNT);
-        float g[4];
-        if (BF16G) {
-            g[0] = bf16_to_f32((uint32_t)gw[0] & 0xFFFFu);
-            g[1] = bf16_to_f32((uint32_t)gw[0] >> 16);
-            g[2] = bf16_to_f32((uint32_t)gw[1] & 0xFFFFu);
-            g[3] = bf16_to_f32((uint32_t)gw[1] >> 16);
-        } else {
+    // g (and the fold's accumulator), m and v are loaded ahead of p: the
+    // moments need only those, and m and v are stored before the sqrt
+    // and the division that p waits for (C1, alternating fresh
+    // processes, against loading p first and storing p, m, v after both
+    // halves: faster in 8 of 8 pairs in two sessions, 0.4-0.6 %, and
+    // even in a third)
+    i32x2 gw = {0, 0};
+    i32x4 ga = {0, 0, 0, 0}, A = {0, 0, 0, 0};
+    if (BF16G) gw = __builtin_amdgcn_raw_buffer_load_b64(s.rg, o * 2, 0, kBufNT);
+    else ga = __builtin_amdgcn_raw_buffer_load_b128(s.rg, o * 4, 0, kBufNT);
+    if (FOLD) A = __builtin_amdgcn_raw_buffer_load_b128(s.ra, o * 4, 0, kBufNT);
+    const i32x4 M = __builtin_amdgcn_raw_buffer_load_b128(s.rm, o * 4, 0, kBufNT);
+    const i32x4 V = __builtin_amdgcn_raw_buffer_load_b128(s.rv, o * 4, 0, kBufNT);
+    const i32x4 P = __builtin_amdgcn_raw_buffer_load_b128(s.rp, o * 4, 0, kBufNT);
+    float g[4];
+    if (BF16G) {
+        g[0] = bf16_to_f32((uint32_t)gw[0] & 0xFFFFu);
+        g[1] = bf16_to_f32((uint32_t)gw[0] >> 16);
+        g[2] = bf16_to_f32((uint32_t)gw[1] & 0xFFFFu);
+        g[3] = bf16_to_f32((uint32_t)gw[1] >> 16);
+    } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) g[j] = __int_as_float(ga[j]);
-        }
-        if (FOLD) {
-            // the last microbatch folded in: acc + widen(g), one fp32 rounding
+        for (int j = 0; j < 4; ++j) g[j] = __int_as_float(ga[j]);
+    }
+    if (FOLD) {
+        // the last microbatch folded in: acc + widen(g), one fp32 rounding
 #pragma unroll
-            for (int j = 0; j < 4; ++j) g[j] = __int_as_float(A[j]) + g[j];
-        }
-        float p[4], m[4], v[4];
+        for (int j = 0; j < 4; ++j) g[j] = __int_as_float(A[j]) + g[j];
+    }
+    float p[4], m[4], v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            m[j] = __int_as_float(M[j]);
-            v[j] = __int_as_float(V[j]);
-            Op::moments(g[j], m[j], v[j], c, coef);
-        }
-        __builtin_amdgcn_raw_buffer_store_b128(bits4(m), rm, o * 4, 0, kBufNT);
-        __builtin_amdgcn_raw_buffer_store_b128(bits4(v), rv, o * 4, 0, kBufNT);
+    for (int j = 0; j < 4; ++j) {
+        m[j] = __int_as_float(M[j]);
+        v[j] = __int_as_float(V[j]);
+        Op::moments(g[j], m[j], v[j], c, coef);
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(bits4(m), s.rm, o * 4, 0, kBufNT);
+    __builtin_amdgcn_raw_buffer_store_b128(bits4(v), s.rv, o * 4, 0, kBufNT);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            p[j] = __int_as_float(P[j]);
-            Op::param(p[j], m[j], v[j], c);
-        }
-        __builtin_amdgcn_raw_buffer_store_b128(bits4(p), rp, o * 4, 0, kBufNT);
-        if (d.copy) {
-            const i32x2 w = {(int32_t)(f32_to_bf16(p[0]) | (f32_to_bf16(p[1]) << 16)),
-                             (int32_t)(f32_to_bf16(p[2]) | (f32_to_bf16(p[3]) << 16))};
-            __builtin_amdgcn_raw_buffer_store_b64(w, rc, o * 2, 0, kBufNT);
-        }
+    for (int j = 0; j < 4; ++j) {
+        p[j] = __int_as_float(P[j]);
+        Op::param(p[j], m[j], v[j], c);
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(bits4(p), s.rp, o * 4, 0, kBufNT);
+    if (has_copy) {
+        const i32x2 w = {(int32_t)(f32_to_bf16(p[0]) | (f32_to_bf16(p[1]) << 16)),
+                         (int32_t)(f32_to_bf16(p[2]) | (f32_to_bf16(p[3]) << 16))};
+        __builtin_amdgcn_raw_buffer_store_b64(w, s.rc, o * 2, 0, kBufNT);
     }
 }
 
@@ -645,12 +696,19 @@ __device__ __forceinline__ void adam_range(const AdamDesc& d, const ely_adamw_co
                                            int64_t e1) {
     using Op = AdamOp<BF16G, ORDER, WD, CLIP, FOLD>;
     int64_t done = e0;
-    if (d.aligned) {
-        const int64_t steps = (e1 - e0) / kStep;
-        if (steps > 0) adam_steps<BF16G, ORDER, WD, CLIP, FOLD>(d, c, coef, e0, steps);
-        done = e0 + steps * kStep;
+    if (d.vec) {
+        const int32_t ne = (int32_t)(e1 - e0);  // a tile's range: at most kAdamTile elements
+        const AdamStreams<BF16G, FOLD> s(d, e0, ne);
+        int32_t o = (int32_t)threadIdx.x * 4;  // the lane's first element
+        int32_t whole = ne / (int32_t)kStep * (int32_t)kStep;
+        for (int32_t b = 0; b < whole; b += (int32_t)kStep)
+            adam_quad<BF16G, ORDER, WD, CLIP, FOLD>(s, d.copy != nullptr, c, coef, b + o);
+        if (whole == ne) return;
+        // a tensor's last, partial step: its whole quads, then the elements left over below
+        if (whole + o + 4 <= ne) adam_quad<BF16G, ORDER, WD, CLIP, FOLD>(s, d.copy != nullptr, c, coef, whole + o);
+        done = e0 + ne / 4 * 4;
     }
-    // Scalar path: unaligned tensors entirely, aligned tensors' last partial step.
+    // Scalar path: the last elements of a tensor, or all of one off its elements' addresses.
     for (int64_t i = done + threadIdx.x; i < e1; i += kAdamBlock) {
         float p = *gp(d.p + i), m = *gp(d.m + i), v = *gp(d.v + i);
         float g = BF16G ? bf16_to_f32(*gp(static_cast<const uint16_t*>(d.g) + i)) : *gp(static_cast<const float*>(d.g) + i);
@@ -804,7 +862,7 @@ static NormLaunch grad_norm_impl(const ely_tensor* accs, const ely_tensor* grads
         d.numel = grads[i].numel;
         d.tile_begin = tiles;
         d.dtype = grads[i].dtype;
-        d.aligned = aligned16(grads[i].ptr) && (!accs || aligned16(accs[i].ptr)) ? 1 : 0;
+        d.vec = elem_aligned(grads[i].ptr, d.dtype) && (!accs || elem_aligned(accs[i].ptr, ELY_F32)) ? 1 : 0;
         table.push_back(d);
         tiles += (d.numel + tile - 1) / tile;
     }
@@ -940,8 +998,8 @@ static void adamw_impl(const ely_tensor* params, const ely_tensor* accs, const e
         d.copy = copies ? static_cast<uint16_t*>(copies[i].ptr) : nullptr;
         d.numel = ne;
         d.tile_begin = (int32_t)tiles;
-        d.aligned = aligned16(d.p) && aligned16(d.g) && aligned16(d.m) && aligned16(d.v) &&
-                    (!d.copy || aligned16(d.copy)) && (!d.acc || aligned16(d.acc));
+        d.vec = elem_aligned(d.p, ELY_F32) && elem_aligned(d.g, gdt) && elem_aligned(d.m, ELY_F32) &&
+                elem_aligned(d.v, ELY_F32) && elem_aligned(d.copy, ELY_BF16) && elem_aligned(d.acc, ELY_F32);
         table.push_back(d);
         cs.push_back(consts[i]);
         tiles += (ne + kAdamTile - 1) / kAdamTile;
@@ -1074,7 +1132,7 @@ int ely_scale_inplace(const ely_tensor* ts, int32_t n, const float* coef_dev, vo
             d.numel = ts[i].numel;
             d.tile_begin = nl.tiles;
             d.dtype = ts[i].dtype;
-            d.aligned = aligned16(ts[i].ptr) ? 1 : 0;
+            d.vec = elem_aligned(ts[i].ptr, d.dtype) ? 1 : 0;
             nl.args.d[nl.entries++] = d;
             nl.tiles += (d.numel + tile - 1) / tile;
             nl.dt = nl.dt == -2 ? d.dtype : (nl.dt == d.dtype ? nl.dt : -1);

@@ -128,3 +128,61 @@ def test_cast_fold_and_widen_at_any_address(n):
             want[off : off + n] = (acc[off : off + n].float() + part[1 : n + 1].float()).to(acc.dtype)
             pieces.fold_add(got[off : off + n], part[1 : n + 1])
             assert torch.equal(got, want)
+
+
+# lengths around a quad, a wave's step, an 8-element group, both norm tiles
+LENGTHS = [1, 2, 3, 4, 5, 7, 8, 9, 63, 255, 256, 257, 511, 513, 4095, 4096, 4097, 12291, 16385]
+
+
+def _lay(values, packed):
+    """The values as views of one buffer, back to back from element 1 on, or
+    each in memory of its own."""
+    if not packed:
+        return [v.clone() for v in values]
+    flat = torch.empty(1 + sum(v.numel() for v in values), dtype=values[0].dtype, device="cuda")
+    out, o = [], 1
+    for v in values:
+        out.append(flat[o : o + v.numel()])
+        out[-1].copy_(v)
+        o += v.numel()
+    return out
+
+
+@pytest.mark.parametrize("gdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("order,fold", [("host", False), ("torch", True)])
+def test_packed_step_equals_the_step_over_separate_tensors(gdt, order, fold):
+    """Neighbours in one buffer: a lane past its tensor's end would change
+    the next tensor's values."""
+    from elysium_wan_amd import optim
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda scale: [torch.randn(n, generator=g, device="cuda") * scale for n in LENGTHS]  # noqa: E731
+    p, acc, gr = rnd(0.02), rnd(1e-3), [t.to(gdt) for t in rnd(1e-1)]
+    got = []
+    for packed in (False, True):
+        say("packed step", gdt, order, fold, packed)
+        ps = [t.requires_grad_(True) for t in _lay(p, packed)]
+        copies = _lay([torch.zeros(n, dtype=torch.bfloat16, device="cuda") for n in LENGTHS], packed)
+        opt = optim.FusedAdamW(ps, lr=3e-4, weight_decay=0.1, order=order, max_norm=1.0, working_copy=copies)
+        for _ in range(2):
+            opt.step(grads=_lay(gr, packed), acc=_lay(acc, packed) if fold else None)
+        got.append([t.detach() for t in ps] + copies + [opt.state[i][k] for i in range(len(ps)) for k in ("exp_avg", "exp_avg_sq")] + [opt.grad_norm()])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("gdt", [torch.bfloat16, torch.float32])
+def test_packed_clip_equals_the_clip_over_separate_tensors(gdt):
+    from elysium_wan_amd import optim
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    values = [(torch.randn(n, generator=g, device="cuda") * 0.1).to(gdt) for n in LENGTHS * 3]  # past the argument table too
+    got = []
+    for packed in (False, True):
+        say("packed clip", gdt, packed)
+        ps = [torch.zeros_like(v) for v in values]
+        for t, v in zip(ps, _lay(values, packed)):
+            t.grad = v
+        got.append([optim.clip_grad_norm_(ps, 1.0)] + [t.grad for t in ps])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
