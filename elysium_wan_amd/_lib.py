@@ -15,6 +15,11 @@ import threading
 import numpy as np
 import torch
 
+try:
+    from . import _native
+except ImportError as e:  # not built yet: load_native() says so at the first call
+    _native, _native_error = None, e
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libelyhip.so")
 
@@ -141,6 +146,17 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return _lib
 
 
+def load_native():
+    """The module of the plain calls (csrc/binding.cpp); raises RuntimeError
+    when it has not been built."""
+    if _native is None:
+        raise RuntimeError(
+            f"elysium_wan_amd._native cannot be loaded ({_native_error}): build the HIP library first "
+            "(python -m elysium_wan_amd.build, or __graft_entry__.build())"
+        )
+    return _native
+
+
 def check(status: int, what: str) -> None:
     if status == OK:
         return
@@ -224,20 +240,12 @@ def stream_ptr(device: torch.device) -> int:
 
 # ---------------------------------------------------------------- workspace
 
-_ws: dict = {}
-_ws_lock = threading.Lock()
-
 
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """A scratch byte buffer of at least nbytes, one per (device, current
-    stream).  Calls on one stream are ordered, so reuse is safe; when it
-    grows, the old buffer returns to torch's allocator, which reuses it only
-    after work already queued on that stream."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    nbytes = max(int(nbytes), 256)
-    with _ws_lock:
-        buf = _ws.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-            _ws[key] = buf
-        return buf
+    stream), shared with the plain calls of csrc/binding.cpp.  Calls on one
+    stream are ordered, so reuse is safe; when it grows, the old buffer
+    returns to torch's allocator, which reuses it only after work already
+    queued on that stream."""
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return load_native().workspace(index, int(nbytes))

@@ -4,6 +4,8 @@
 
 Every csrc/*.hip translation unit is compiled by hipcc for gfx950 only and
 linked into elysium_wan_amd/libelyhip.so, which the package loads with ctypes.
+csrc/binding.cpp (host code against torch's headers) becomes
+elysium_wan_amd/_native.so beside it, the plain calls' way into that library.
 Flags that matter for the numerics:
 
 * -ffp-contract=off: no fused multiply-add unless the source writes one, so
@@ -23,11 +25,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libelyhip.so")
+NATIVE = os.path.join(HERE, "_native.so")
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -64,15 +68,48 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_native() -> str:
+    """csrc/binding.cpp to an object file, with the host compiler."""
+    import torch
+
+    obj = os.path.join(BUILD, "binding.cpp.o")
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    cmd = [
+        "g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{inc}", f"-I{os.path.join(inc, 'torch', 'csrc', 'api', 'include')}", f"-I{sysconfig.get_paths()['include']}",
+        f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}",
+        "-c", os.path.join(CSRC, "binding.cpp"), "-o", obj,
+    ]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on binding.cpp:\n{r.stdout}\n{r.stderr}")
+    return obj
+
+
+def _link_native(obj: str) -> None:
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = NATIVE + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{HERE}", "-lelyhip", f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link of _native.so failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, NATIVE)
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every csrc/*.hip for gfx950 and link libelyhip.so (always
-    rebuilds).  Returns the library path."""
+    """Compile every csrc/*.hip for gfx950 and link libelyhip.so, then
+    _native.so against it (always rebuilds).  Returns the library path."""
     os.makedirs(BUILD, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     jobs = min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
     with cf.ThreadPoolExecutor(jobs) as ex:
+        native = ex.submit(_compile_native)
         objs = list(ex.map(_compile, srcs))
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
@@ -80,6 +117,7 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    _link_native(native.result())
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources", file=sys.stderr)
     return LIB

@@ -121,6 +121,10 @@ def quantize(x: torch.Tensor, fmt: str = "e4m3", per_tensor: bool = False, k_hin
     right, x is read once instead of twice.  Without one, a per-tensor x of
     64 MiB or more guesses its exponent from a sample of x (every 61st
     2,048-element segment) and is read once when the guess holds."""
+    if k_hint is None:
+        done = _lib.load_native().quantize(x, fmt, per_tensor)
+        if done is not None:
+            return done
     f = _fmt(fmt)
     hint = _hint(k_hint, per_tensor, "quantize")
     if hint is not None:
@@ -155,6 +159,10 @@ def _fmt_of(q: torch.Tensor) -> str:
 def dequantize(q: torch.Tensor, k: torch.Tensor, dtype: torch.dtype = torch.float32) -> torch.Tensor:
     """q.to(dtype) * 2^k, exact (model/fp8.py:52-53).  k holds one exponent
     per row of q (shape [..., 1], or one element for a per-tensor q)."""
+    if dtype is torch.bfloat16 or dtype is torch.float32:
+        done = _lib.load_native().dequantize(q, k, dtype is torch.bfloat16)
+        if done is not None:
+            return done
     fmt = _fmt_of(q)
     _lib.require_gpu(q, "dequantize")
     if dtype not in (torch.float32, torch.bfloat16):
@@ -182,6 +190,10 @@ def dequantize(q: torch.Tensor, k: torch.Tensor, dtype: torch.dtype = torch.floa
 def roundtrip(x: torch.Tensor, fmt: str = "e4m3", per_tensor: bool = False, k_hint: int | torch.Tensor | None = None) -> torch.Tensor:
     """The declared recipe at a boundary: quantize then dequantize, in x's
     dtype (model/fp8.py:56-63), fused into one pass.  k_hint as quantize's."""
+    if k_hint is None:
+        done = _lib.load_native().roundtrip(x, fmt, per_tensor)
+        if done is not None:
+            return done
     f = _fmt(fmt)
     hint = _hint(k_hint, per_tensor, "roundtrip")
     if hint is not None:

@@ -431,7 +431,6 @@ class FusedAdamW:
             return host_consts(lr, betas, eps, weight_decay, t)
         return torch_consts(lr, betas, eps, weight_decay, t)
 
-    @torch.no_grad()
     def step(self, on_param=None, grads=None, acc=None) -> None:
         """One AdamW step over every parameter with a gradient, in order;
         `on_param(i)` runs right after parameter i's update is issued
@@ -449,6 +448,38 @@ class FusedAdamW:
         earlier microbatches; the step's gradient is then acc[i] + grads[i]
         rounded once to fp32 (pieces.fold_add), folded inside the update
         without writing acc."""
+        if on_param is not None or not self._plain_step(grads, acc):
+            self._any_step(on_param, grads, acc)
+
+    def _plain_step(self, grads, acc) -> bool:
+        """The step of a shard of ordinary tensors whose state is in place,
+        with moments in HBM, in one native call (csrc/binding.cpp): the same
+        checks, tables and launches as _any_step.  False, with nothing done,
+        for any other."""
+        dev = self.device
+        if self.moments != "device" or dev is None or dev.index is None or self._steps is None:
+            return False
+        gl = [p.grad for p in self.params] if grads is None else list(grads) if type(grads) is tuple else grads
+        acc = list(acc) if type(acc) is tuple else acc
+        lr, betas, eps, wd = self._hyper()
+        norm = self._norm
+        if self.max_norm is not None and (norm is None or norm.device != dev):
+            norm = torch.empty(16, dtype=torch.uint8, device=dev)
+        done = _lib.load_native().adamw_step(
+            self.params, gl, acc, self._st, self._steps, self.working_copies, dev.index,
+            _lib.ORDER_HOST if self.order == "host" else _lib.ORDER_TORCH, int(wd != 0), self.max_norm, norm,
+            lambda t: self._consts(t, lr, betas, eps, wd),
+        )
+        if done is None:
+            return False
+        if self.max_norm is not None:
+            self._norm = norm
+        rc, call = done
+        _lib.check(rc, f"{self.recipe} step" if call else "grad norm")
+        return True
+
+    @torch.no_grad()
+    def _any_step(self, on_param, grads, acc) -> None:
         if grads is not None and len(grads) != len(self.params):
             raise ValueError(f"{len(grads)} gradients for {len(self.params)} parameters")
         if acc is not None and len(acc) != len(self.params):
@@ -938,8 +969,11 @@ def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0, error_i
     fp32 total norm as a device tensor."""
     if norm_type != 2.0:
         raise ValueError("clip_grad_norm_ on MI355X computes the 2-norm only")
-    if isinstance(parameters, torch.Tensor):
-        parameters = [parameters]
+    parameters = [parameters] if isinstance(parameters, torch.Tensor) else list(parameters)
+    if not error_if_nonfinite:
+        total = _lib.load_native().clip(parameters, max_norm)
+        if total is not None:
+            return total
     grads = [p.grad for p in parameters if p.grad is not None]
     if not grads:
         return torch.tensor(0.0)

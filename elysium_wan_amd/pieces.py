@@ -23,6 +23,9 @@ from . import optim as _optim
 def cast_piece(p: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """runtime/pieces.py:192-195: a new tensor, never an alias of the master."""
     if dtype == torch.bfloat16 and p.dtype == torch.float32:
+        done = _lib.load_native().cast_bf16(p)
+        if done is not None:
+            return done
         _lib.require_gpu(p, "cast_piece")
         src = p.detach().contiguous()
         out = torch.empty(src.shape, dtype=torch.bfloat16, device=src.device)
@@ -45,6 +48,9 @@ def fold_start(g: torch.Tensor) -> torch.Tensor:
     if g.dtype == torch.float32:
         return g.detach().clone()
     # widening is exact: the fp32 value of a bf16 is its bits moved to the top
+    done = _lib.load_native().widen_bf16(g)
+    if done is not None:
+        return done
     src = g.detach().contiguous()
     out = torch.empty(src.shape, dtype=torch.float32, device=src.device)
     L = _lib.load()
@@ -57,6 +63,8 @@ def fold_add(acc: torch.Tensor, g: torch.Tensor) -> None:
     element.  An accumulator that is not fold_start's fp32 (a bf16 one) takes
     the reference's in-place add as torch computes it there: the fp32 sum
     rounded to bf16 (ely_fold_add_bf16)."""
+    if _lib.load_native().fold_add(acc, g) is not None:
+        return
     if acc.dtype == torch.int64:
         if g.dtype != torch.int64:
             raise ValueError(f"a count lane folds int64 only, got {g.dtype}")

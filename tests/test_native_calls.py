@@ -1,0 +1,124 @@
+"""The native calls (csrc/binding.cpp) decline what is no plain call, before
+any effect, so that the Python code behind them answers as it always did."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from elysium_wan_amd import _lib
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def _declined(x):
+    N = _lib.load_native()
+    return [N.quantize(x, "e4m3", False), N.roundtrip(x, "e4m3", True), N.cast_bf16(x), N.widen_bf16(x), N.fold_add(x, x),
+            N.dequantize(x, x, True), N.clip([x], 1.0)]
+
+
+def test_host_tensors_and_other_objects_are_declined():
+    for x in (torch.zeros(3, 8), torch.zeros(3, 8, dtype=torch.float16), None, 3.0, "x"):
+        assert all(r is None for r in _declined(x))
+    p = torch.zeros(4)
+    args = [[p], [torch.ones(4)], None, {}, torch.zeros(1), None, 0, 0, 0, None, None, lambda t: [0.0] * 8]
+    assert _lib.load_native().adamw_step(*args) is None and float(args[4][0]) == 0.0
+
+
+@pytest.mark.gpu
+def test_plain_calls_are_taken_and_equal_the_python_path(monkeypatch):
+    from elysium_wan_amd import fp8, optim, pieces
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(33, 1001, generator=g, device="cuda").bfloat16()
+    long = torch.randn(1, 70001, generator=g, device="cuda")
+
+    def calls():
+        q, k = fp8.quantize(x)
+        ql, kl = fp8.quantize(long, "e5m2", per_tensor=True)
+        acc = x.float()
+        pieces.fold_add(acc, x)
+        h = x.clone()
+        pieces.fold_add(h, x)
+        ps = [x.float().requires_grad_(True), long.clone().requires_grad_(True)]
+        opt = optim.FusedAdamW(ps, lr=1e-3, weight_decay=0.1, max_norm=1.0, working_copy=True)
+        for gs in ([x, long], [None, long.bfloat16()], [x.float(), long.bfloat16()]):  # state made, one skipped, two dtypes
+            opt.step(grads=gs)
+            opt.step(grads=tuple(gs), acc=[torch.ones_like(p) for p in ps])
+        cs = [torch.zeros_like(long), torch.zeros_like(x), torch.zeros(3, device="cuda")]
+        cs[0].grad, cs[1].grad = long.clone(), x.clone()
+        total = optim.clip_grad_norm_(iter(cs), 0.5)
+        return [q.view(torch.uint8), k, ql.view(torch.uint8), kl, fp8.roundtrip(x, "e5m2"), fp8.roundtrip(long, per_tensor=True),
+                fp8.dequantize(q, k), fp8.dequantize(ql, kl, torch.bfloat16), pieces.cast_piece(long, torch.bfloat16),
+                pieces.fold_start(x), acc, h, *[p.detach() for p in ps], *opt.working_copies, opt.grad_norm(),
+                *[opt.state[i][n] for i in (0, 1) for n in ("step", "exp_avg", "exp_avg_sq")], total, cs[0].grad, cs[1].grad]
+
+    N = _lib.load_native()
+    taken = []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(N, name)
+
+            def call(*a):
+                r = f(*a)
+                taken.append((name, r is not None))
+                return r
+
+            return f if name == "workspace" else call
+
+    class Off:
+        workspace = staticmethod(N.workspace)
+
+        def __getattr__(self, name):
+            return lambda *a: None
+
+    monkeypatch.setattr(_lib, "_native", Spy())
+    fast = calls()
+    # all but the optimizer's first step, which makes its state, go the native way
+    assert [t for t in taken if not t[1]] == [("adamw_step", False)] or not [t for t in taken if not t[1]]
+    assert {n for n, ok in taken if ok} == {"quantize", "roundtrip", "dequantize", "cast_bf16", "widen_bf16", "fold_add", "adamw_step", "clip"}
+    monkeypatch.setattr(_lib, "_native", Off())
+    slow = calls()
+    for a, b in zip(fast, slow):
+        assert a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_views_wrappers_and_modes_are_declined():
+    from torch.overrides import TorchFunctionMode
+
+    x = torch.randn(16, 32, device="cuda").bfloat16()
+    N = _lib.load_native()
+    for y in (x.t(), x.to(torch.float16), x[0, 0], x[:0], x.as_subclass(_Sub), x.cpu()):
+        assert N.quantize(y, "e4m3", False) is None and N.roundtrip(y, "e4m3", False) is None
+    assert N.quantize(x, "e3m4", False) is None and N.quantize(x, 3, False) is None
+    assert N.fold_add(x.float().t(), x) is None and N.fold_add(x.float(), x[:3]) is None
+    q, k = N.quantize(x, "e4m3", False)
+    assert N.dequantize(q, k[:3], True) is None and N.dequantize(q, k.long(), True) is None and N.dequantize(x, k, True) is None
+    seen = []
+    torch.vmap(lambda row: seen.append(N.roundtrip(row, "e4m3", False)) or row * 1)(x)
+    with TorchFunctionMode():
+        seen.append(N.quantize(x, "e4m3", False))
+    with torch._subclasses.FakeTensorMode(allow_non_fake_inputs=True):
+        seen.append(N.quantize(x, "e4m3", False))
+    assert seen == [None, None, None]
+
+
+@pytest.mark.gpu
+def test_a_failed_check_leaves_state_and_tensors_alone():
+    """The native step looks every tensor over before it counts a step."""
+    from elysium_wan_amd import optim
+
+    ps = [torch.ones(300, device="cuda", requires_grad=True) for _ in range(3)]
+    opt = optim.FusedAdamW(ps, lr=1e-3, max_norm=1.0)
+    good = [torch.ones(300, device="cuda") for _ in ps]
+    opt.step(grads=good)
+    before = [p.detach().clone() for p in ps]
+    for bad in (torch.ones(299, device="cuda"), torch.ones(600, device="cuda")[::2], torch.ones(300), torch.ones(300, device="cuda").half()):
+        with pytest.raises(ValueError):
+            opt.step(grads=good[:2] + [bad])
+        assert [float(opt.state[i]["step"]) for i in range(3)] == [1.0] * 3
+        assert all(torch.equal(p.detach(), b) for p, b in zip(ps, before))
