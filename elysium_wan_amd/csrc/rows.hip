@@ -9,8 +9,8 @@
 //   acc[idx[j]] += a[rows_a[j]] + 0.0                  (later, free rows)
 //   acc[idx[j]]  = a[j] + e_j       / acc[idx[j]] += a[j] + e_j
 //                                                      (held rows resolved)
-// over a set of distinct rows, which this kernel runs: one block per row
-// (strided), 16-byte vectors across the row when it is aligned.  e_j is the
+// over a set of distinct rows, which this kernel runs: a wave per piece of a
+// row, 16-byte vectors across it.  e_j is the
 // embedding row b[b_rows[j]] of a held row the microbatch touched, +0.0 for
 // one it did not (b_rows[j] < 0), or b[j] of a compact b.  A second kernel
 // takes a whole Head gradient in one pass: its free rows fold, its held
@@ -25,12 +25,33 @@
 namespace ely {
 namespace {
 
-constexpr int kRowBlock = 256;
-// one block per row up to this many; longer lists stride
-constexpr int64_t kRowGrid = 1 << 16;
+// A wave moves V 16-byte vectors per lane of a row and ends, a row's pieces
+// across the grid, rows down (a longer list strides).  Launches that touch
+// more than the 256 MB MALL holds stream (nontemporal loads, and the split's
+// stores); the others keep to plain loads, for the rows and the sum are read
+// again soon.  Against a 256-thread block per row, in one process on the same
+// buffers, a third of the rows held: 32,768 x 2,560 fp32 split 170 -> 142 us
+// (5.3 -> 6.3 TB/s) and fold of the held 77 -> 61, bf16 84 -> 74 and 32 -> 32,
+// 8,192 x 1,024 fp32 14.4 both and 7.0 -> 7.6; 32,768 x 1,001 bf16, element
+// by element before, 89 -> 40 and 27 -> 17.
+constexpr int kSplitVecs = 2, kFoldVecs = 1;
+constexpr int64_t kMallBytes = (int64_t)256 << 20;
+constexpr int64_t kRowGrid = 65535;
 
-typedef float rf4 __attribute__((ext_vector_type(4)));
 typedef uint32_t ru4 __attribute__((ext_vector_type(4)));
+// ... at any element's address (see the codec's vector types)
+typedef uint32_t ru4u __attribute__((ext_vector_type(4), aligned(2)));
+#define ROWS_G1 __attribute__((address_space(1)))
+template <bool NT>
+__device__ __forceinline__ ru4 ld_row(const void* p) {
+    if (NT) return __builtin_nontemporal_load((const ROWS_G1 ru4u*)p);
+    return *(const ROWS_G1 ru4u*)p;
+}
+template <bool NT>
+__device__ __forceinline__ void st_row(void* p, ru4 v) {
+    if (NT) __builtin_nontemporal_store((ru4u)v, (ROWS_G1 ru4u*)p);
+    else *(ROWS_G1 ru4u*)p = v;
+}
 
 // v = a + b (b = +0.0 when absent) rounded to the dtype, then acc = v or
 // acc + v rounded to the dtype: torch's two elementwise adds.
@@ -43,8 +64,6 @@ __device__ __forceinline__ float fold1(float acc, float a, float b, bool first) 
     if (BF16) s = bf16_to_f32(f32_to_bf16(s));
     return s;
 }
-
-constexpr int kRowUnroll = 4;  // 16-byte vectors per thread loaded before the first is stored
 
 // One vector of 4 fp32 or 8 bf16 elements: acc (=|+=) x + y, each add rounded
 // to the dtype (y = 0 when the row has no b).
@@ -64,114 +83,114 @@ __device__ __forceinline__ ru4 fold_vec(ru4 z, ru4 x, ru4 y, int first) {
     return o;
 }
 
-// One row of d elements: ac (=|+=) av + (bv or +0.0).  Aligned rows move
-// 16-byte vectors, kRowUnroll per thread loaded before any is stored, so a
-// row's loads are in flight together; others go element by element.
-template <bool BF16>
-__device__ __forceinline__ void fold_row(void* ac_, const void* av_, const void* bv_, int64_t d, int first, int vec) {
-    if (vec) {
-        const int64_t nvec = d / (BF16 ? 8 : 4);
-        ru4* ac = static_cast<ru4*>(ac_);
-        const ru4* av = static_cast<const ru4*>(av_);
-        const ru4* bv = static_cast<const ru4*>(bv_);
-        for (int64_t v0 = threadIdx.x; v0 < nvec; v0 += (int64_t)kRowBlock * kRowUnroll) {
-            ru4 x[kRowUnroll], y[kRowUnroll], z[kRowUnroll];
+// Piece `piece` of one row of d elements: ac (=|+=) av + (bv or +0.0), its
+// vectors' loads all issued before the first is stored.  The row's last
+// elements, short of a vector, go to the last piece's lanes, one each.
+template <bool BF16, int V, bool NTL, bool NTS>
+__device__ __forceinline__ void fold_piece(char* ac, const char* av, const char* bv, int64_t d, int piece, int first,
+                                           int vec) {
+    constexpr int EPV = BF16 ? 8 : 4, ESZ = BF16 ? 2 : 4;
+    const int64_t nvec = vec ? d / EPV : 0;
+    const int64_t v0 = (int64_t)piece * (kWave * V) + threadIdx.x;
+    ru4 x[V], y[V], z[V];
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u) {
-                const int64_t v = v0 + (int64_t)u * kRowBlock;
-                const ru4 zero = {0u, 0u, 0u, 0u};
-                x[u] = v < nvec ? av[v] : zero;
-                y[u] = (v < nvec && bv) ? bv[v] : zero;
-                z[u] = (v < nvec && !first) ? ac[v] : zero;
-            }
+    for (int u = 0; u < V; ++u) {
+        const int64_t v = v0 + u * kWave;
+        const ru4 zero = {0u, 0u, 0u, 0u};
+        x[u] = v < nvec ? ld_row<NTL>(av + v * 16) : zero;
+        y[u] = (v < nvec && bv) ? ld_row<NTL>(bv + v * 16) : zero;
+        z[u] = (v < nvec && !first) ? ld_row<NTL>(ac + v * 16) : zero;
+    }
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u) {
-                const int64_t v = v0 + (int64_t)u * kRowBlock;
-                if (v < nvec) ac[v] = fold_vec<BF16>(z[u], x[u], y[u], first);
-            }
-        }
-    } else if (BF16) {
-        uint16_t* ac = static_cast<uint16_t*>(ac_);
-        const uint16_t* av = static_cast<const uint16_t*>(av_);
-        const uint16_t* bv = static_cast<const uint16_t*>(bv_);
-        for (int64_t c = threadIdx.x; c < d; c += kRowBlock) {
-            const float z = first ? 0.0f : bf16_to_f32(ac[c]);
-            ac[c] = (uint16_t)f32_to_bf16(fold1<true>(z, bf16_to_f32(av[c]), bv ? bf16_to_f32(bv[c]) : 0.0f, first));
-        }
-    } else {
-        float* ac = static_cast<float*>(ac_);
-        const float* av = static_cast<const float*>(av_);
-        const float* bv = static_cast<const float*>(bv_);
-        for (int64_t c = threadIdx.x; c < d; c += kRowBlock) {
-            const float z = first ? 0.0f : ac[c];
-            ac[c] = fold1<false>(z, av[c], bv ? bv[c] : 0.0f, first);
+    for (int u = 0; u < V; ++u) {
+        const int64_t v = v0 + u * kWave;
+        if (v < nvec) st_row<NTS>(ac + v * 16, fold_vec<BF16>(z[u], x[u], y[u], first));
+    }
+    if (piece != (int)gridDim.x - 1) return;
+    for (int64_t c = nvec * EPV + threadIdx.x; c < d; c += kWave) {
+        if (BF16) {
+            uint16_t* o = reinterpret_cast<uint16_t*>(ac) + c;
+            const float z1 = first ? 0.0f : bf16_to_f32(*o);
+            *o = (uint16_t)f32_to_bf16(fold1<true>(z1, bf16_to_f32(reinterpret_cast<const uint16_t*>(av)[c]),
+                                                  bv ? bf16_to_f32(reinterpret_cast<const uint16_t*>(bv)[c]) : 0.0f, first));
+        } else {
+            float* o = reinterpret_cast<float*>(ac) + c;
+            *o = fold1<false>(first ? 0.0f : *o, reinterpret_cast<const float*>(av)[c],
+                              bv ? reinterpret_cast<const float*>(bv)[c] : 0.0f, first);
         }
     }
 }
 
-template <bool BF16>
-__global__ __launch_bounds__(kRowBlock) void rows_fold_kernel(void* __restrict__ acc, const void* __restrict__ a,
-                                                              const int64_t* __restrict__ a_rows,
-                                                              const void* __restrict__ b,
-                                                              const int64_t* __restrict__ b_rows,
-                                                              const int64_t* __restrict__ idx, int64_t n_idx,
-                                                              int64_t n_rows, int64_t a_total, int64_t b_total,
-                                                              int64_t d, int first, int vec) {
+template <bool BF16, bool NT>
+__global__ __launch_bounds__(kWave) void rows_fold_kernel(void* __restrict__ acc, const void* __restrict__ a,
+                                                          const int64_t* __restrict__ a_rows,
+                                                          const void* __restrict__ b,
+                                                          const int64_t* __restrict__ b_rows,
+                                                          const int64_t* __restrict__ idx, int64_t n_idx,
+                                                          int64_t n_rows, int64_t a_total, int64_t b_total,
+                                                          int64_t d, int first, int vec) {
     const int64_t esz = BF16 ? 2 : 4;
-    for (int64_t j = blockIdx.x; j < n_idx; j += gridDim.x) {
+    for (int64_t j = blockIdx.y; j < n_idx; j += gridDim.y) {
         const int64_t r = idx[j];
         const int64_t ar = a_rows ? a_rows[j] : j;
         const int64_t br = b ? (b_rows ? b_rows[j] : j) : -1;  // < 0: the row adds +0.0
         // the host checks every index; a row outside the tables is skipped, never touched
         if (r < 0 || r >= n_rows || ar < 0 || ar >= a_total || br >= b_total) continue;
-        fold_row<BF16>(static_cast<char*>(acc) + r * d * esz, static_cast<const char*>(a) + ar * d * esz,
-                       br >= 0 ? static_cast<const char*>(b) + br * d * esz : nullptr, d, first, vec);
+        fold_piece<BF16, kFoldVecs, NT, false>(static_cast<char*>(acc) + r * d * esz,
+                                               static_cast<const char*>(a) + ar * d * esz,
+                                               br >= 0 ? static_cast<const char*>(b) + br * d * esz : nullptr, d,
+                                               blockIdx.x, first, vec);
     }
 }
 
-// A row of `bytes` bytes copied bit for bit: 16-byte vectors (kRowUnroll per
-// thread in flight) when both rows are aligned, bytes otherwise.
-__device__ __forceinline__ void copy_row(char* o, const char* x, int64_t bytes, int vec) {
-    if (vec) {
-        const int64_t nvec = bytes / 16;
-        for (int64_t v0 = threadIdx.x; v0 < nvec; v0 += (int64_t)kRowBlock * kRowUnroll) {
-            ru4 t[kRowUnroll];
+// That piece of a row of d elements copied bit for bit.
+template <bool BF16, int V, bool NTL>
+__device__ __forceinline__ void copy_piece(char* o, const char* x, int64_t d, int piece, int vec) {
+    constexpr int EPV = BF16 ? 8 : 4, ESZ = BF16 ? 2 : 4;
+    const int64_t nvec = vec ? d / EPV : 0;
+    const int64_t v0 = (int64_t)piece * (kWave * V) + threadIdx.x;
+    ru4 t[V];
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u) {
-                const int64_t v = v0 + (int64_t)u * kRowBlock;
-                if (v < nvec) t[u] = reinterpret_cast<const ru4*>(x)[v];
-            }
+    for (int u = 0; u < V; ++u)
+        if (v0 + u * kWave < nvec) t[u] = ld_row<NTL>(x + (v0 + u * kWave) * 16);
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u) {
-                const int64_t v = v0 + (int64_t)u * kRowBlock;
-                if (v < nvec) reinterpret_cast<ru4*>(o)[v] = t[u];
-            }
-        }
-    } else {
-        for (int64_t c = threadIdx.x; c < bytes; c += kRowBlock) o[c] = x[c];
-    }
+    for (int u = 0; u < V; ++u)
+        if (v0 + u * kWave < nvec) st_row<true>(o + (v0 + u * kWave) * 16, t[u]);
+    if (piece != (int)gridDim.x - 1) return;
+    for (int64_t c = nvec * 16 + threadIdx.x; c < d * ESZ; c += kWave) o[c] = x[c];
 }
 
-// A Head gradient in one pass, one block per row: a row r with
+// A Head gradient in one pass, a row's pieces across the grid: a row r with
 // slot[r] < 0 is free and takes acc[r] = a[r] + 0.0 (first) or
 // acc[r] + (a[r] + 0.0), each add rounded to the dtype; a held row
 // (slot[r] >= 0) is copied to held_out[slot[r]] bit for bit and acc[r] is
 // left for its resolve.
-template <bool BF16>
-__global__ __launch_bounds__(kRowBlock) void rows_split_kernel(void* __restrict__ acc, const void* __restrict__ a,
+template <bool BF16, bool NT>
+__global__ __launch_bounds__(kWave) void rows_split_kernel(void* __restrict__ acc, const void* __restrict__ a,
                                                                const int32_t* __restrict__ slot,
                                                                void* __restrict__ held_out, int64_t n_rows,
                                                                int64_t n_held, int64_t d, int first, int vec) {
     const int64_t row_bytes = d * (BF16 ? 2 : 4);
-    for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) {
+    for (int64_t r = blockIdx.y; r < n_rows; r += gridDim.y) {
         const int64_t s = slot[r];
         const char* x = static_cast<const char*>(a) + r * row_bytes;
         if (s < 0)
-            fold_row<BF16>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, first, vec);
+            fold_piece<BF16, kSplitVecs, NT, true>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, blockIdx.x, first, vec);
         else if (s < n_held)  // the host numbers the held rows 0..n_held-1
-            copy_row(static_cast<char*>(held_out) + s * row_bytes, x, row_bytes, vec);
+            copy_piece<BF16, kSplitVecs, NT>(static_cast<char*>(held_out) + s * row_bytes, x, d, blockIdx.x, vec);
     }
 }
+
+// The pieces of a row of d elements across, rows down; a dispatch counts its
+// threads in 32 bits.
+dim3 rows_grid(int64_t rows, int64_t d, int64_t esz, int vec, int vecs, const char* what) {
+    const int64_t per = (int64_t)kWave * vecs;
+    const int64_t pieces = vec ? std::max<int64_t>(1, (d * esz / 16 + per - 1) / per) : 1;
+    if (pieces > 0xFFFFFFFFLL / kWave) fail(ELY_EINVAL, std::string(what) + ": rows too long for one launch");
+    return dim3((unsigned)pieces, (unsigned)std::min({rows, kRowGrid, (int64_t)0xFFFFFFFFLL / (kWave * pieces)}));
+}
+
+bool elem_at(const void* p, int64_t esz) { return reinterpret_cast<uintptr_t>(p) % esz == 0; }
 
 }  // namespace
 }  // namespace ely
@@ -190,16 +209,13 @@ extern "C" int ely_rows_fold(void* acc, const void* a, const int64_t* a_rows, co
         if (b_rows && !b) fail(ELY_EINVAL, "ely_rows_fold: b_rows without b");
         if (b && !b_rows && b_total < n_idx) fail(ELY_EINVAL, "ely_rows_fold: a compact b holds one row per index");
         const int64_t esz = dtype == ELY_BF16 ? 2 : 4;
-        const int64_t v = 16 / esz;
-        const int vec = (d % v == 0) && aligned16(acc) && aligned16(a) && (!b || aligned16(b)) ? 1 : 0;
-        const int64_t blocks = std::min<int64_t>(n_idx, kRowGrid);
-        hipStream_t s = static_cast<hipStream_t>(stream);
-        if (dtype == ELY_BF16)
-            hipLaunchKernelGGL(rows_fold_kernel<true>, dim3((unsigned)blocks), dim3(kRowBlock), 0, s, acc, a, a_rows, b,
-                               b_rows, idx, n_idx, n_rows, a_total, b ? b_total : 0, d, first ? 1 : 0, vec);
-        else
-            hipLaunchKernelGGL(rows_fold_kernel<false>, dim3((unsigned)blocks), dim3(kRowBlock), 0, s, acc, a, a_rows, b,
-                               b_rows, idx, n_idx, n_rows, a_total, b ? b_total : 0, d, first ? 1 : 0, vec);
+        const int vec = elem_at(acc, esz) && elem_at(a, esz) && elem_at(b, esz) ? 1 : 0;
+        const dim3 grid = rows_grid(n_idx, d, esz, vec, kFoldVecs, "ely_rows_fold");
+        const bool stream_it = 3 * n_idx * d * esz > kMallBytes;
+        const auto kern = dtype == ELY_BF16 ? (stream_it ? rows_fold_kernel<true, true> : rows_fold_kernel<true, false>)
+                                            : (stream_it ? rows_fold_kernel<false, true> : rows_fold_kernel<false, false>);
+        hipLaunchKernelGGL(kern, grid, dim3(kWave), 0, static_cast<hipStream_t>(stream), acc, a, a_rows, b, b_rows, idx,
+                           n_idx, n_rows, a_total, b ? b_total : 0, d, first ? 1 : 0, vec);
         check_launch("rows_fold_kernel");
     });
 }
@@ -212,16 +228,14 @@ extern "C" int ely_rows_split(void* acc, const void* a, const int32_t* slot, voi
         if (n_held > n_rows) fail(ELY_EINVAL, "ely_rows_split: more held rows than rows");
         if (n_rows == 0 || d == 0) return;
         if (!acc || !a || !slot || (n_held && !held_out)) fail(ELY_EINVAL, "ely_rows_split: null pointer");
-        const int64_t v = dtype == ELY_BF16 ? 8 : 4;
-        const int vec = (d % v == 0) && aligned16(acc) && aligned16(a) && (!n_held || aligned16(held_out)) ? 1 : 0;
-        const int64_t blocks = std::min<int64_t>(n_rows, kRowGrid);
-        hipStream_t s = static_cast<hipStream_t>(stream);
-        if (dtype == ELY_BF16)
-            hipLaunchKernelGGL(rows_split_kernel<true>, dim3((unsigned)blocks), dim3(kRowBlock), 0, s, acc, a, slot,
-                               held_out, n_rows, n_held, d, first ? 1 : 0, vec);
-        else
-            hipLaunchKernelGGL(rows_split_kernel<false>, dim3((unsigned)blocks), dim3(kRowBlock), 0, s, acc, a, slot,
-                               held_out, n_rows, n_held, d, first ? 1 : 0, vec);
+        const int64_t esz = dtype == ELY_BF16 ? 2 : 4;
+        const int vec = elem_at(acc, esz) && elem_at(a, esz) && elem_at(held_out, esz) ? 1 : 0;
+        const dim3 grid = rows_grid(n_rows, d, esz, vec, kSplitVecs, "ely_rows_split");
+        const bool stream_it = 2 * n_rows * d * esz > kMallBytes;
+        const auto kern = dtype == ELY_BF16 ? (stream_it ? rows_split_kernel<true, true> : rows_split_kernel<true, false>)
+                                            : (stream_it ? rows_split_kernel<false, true> : rows_split_kernel<false, false>);
+        hipLaunchKernelGGL(kern, grid, dim3(kWave), 0, static_cast<hipStream_t>(stream), acc, a, slot, held_out, n_rows,
+                           n_held, d, first ? 1 : 0, vec);
         check_launch("rows_split_kernel");
     });
 }

@@ -186,3 +186,30 @@ def test_packed_clip_equals_the_clip_over_separate_tensors(gdt):
         got.append([optim.clip_grad_norm_(ps, 1.0)] + [t.grad for t in ps])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [1, 3, 7, 8, 9, 255, 511, 513, 1025, 1601])
+def test_tied_fold_at_any_width_equals_the_dense_fold(dtype, d):
+    """Widths around a vector, a wave's piece and its last, against the dense
+    fold in torch's ops; a row's elements past its last vector are folded
+    once."""
+    from elysium_wan_amd.accumulate import TiedRowFold
+
+    n, m, t = 67, 4, 9
+    g = torch.Generator(device="cuda").manual_seed(d)
+    hs = [torch.randn(n, d, generator=g, device="cuda").to(dtype) for _ in range(m)]
+    ids = [torch.randperm(n, generator=g, device="cuda")[:t].sort().values for _ in range(m)]
+    es = [torch.randn(t, d, generator=g, device="cuda").to(dtype) for _ in range(m)]
+    say("tied fold width", dtype, d)
+    fold = TiedRowFold(n, range(m))
+    want = None
+    for k in range(m):
+        fold.add_head(k, hs[k], ids[k])
+        if k:
+            fold.add_embed(k - 1, es[k - 1])
+        e = torch.zeros(n, d, dtype=dtype, device="cuda")
+        e[ids[k]] = es[k]
+        want = hs[k] + e if want is None else want + (hs[k] + e)
+    fold.add_embed(m - 1, es[m - 1])
+    assert torch.equal(fold.result(), want)
