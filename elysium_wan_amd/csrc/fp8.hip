@@ -646,11 +646,9 @@ constexpr int kHintBlocks = 256;         // maxima the reduce launch leaves (4 p
 constexpr int kHintFixupWavesPerCU = ELY_HINT_FIXUP_WPC;
 #ifndef ELY_GUESS_MIN_MB
 // per-tensor rows of at least this many MiB of x take the sampled guess.
-// Back to back on N(0, 1) bf16 (a right guess), per call: 8 MiB 16.4-18.1 us
-// against 12.6-16.5 on the split path, 32 MiB 21.4-21.9 against 17.7-18.8,
-// 64 MiB 29.3-29.9 against 28.8-29.5, 128 MiB 45 against 54, 512 MiB 139
-// against 201: the guess's four small launches cost what its saved read wins
-// back near 64 MiB
+// Back to back on N(0, 1) bf16 (a right guess), per call: 64 MiB 24.0 us
+// against 25.3 on the split path, 76 MiB 26.7 against 29.0, 128 MiB 38.8
+// against 47.6, 1 GiB 253 against 386 (of fp32, 128 MiB 35 against 44)
 #define ELY_GUESS_MIN_MB 64
 #endif
 #ifndef ELY_GUESS_STRIDE
@@ -658,80 +656,106 @@ constexpr int kHintFixupWavesPerCU = ELY_HINT_FIXUP_WPC;
 #endif
 constexpr int64_t kGuessStride = ELY_GUESS_STRIDE;
 
-// The hint: k_hint, or *k_hint_dev when that is given (read here, before
-// the fixup launch writes k, which may be the same word); with hint_is_amax,
-// *k_hint_dev holds fp32 |x|max bits (a sample's, guess_amax_kernel) and
-// the hint is their exponent.  Wave 0 keeps the hint it read in hint_copy
-// for the fixup.  A hint outside the instruction path's range converts
-// nothing here: the call is then a miss.
+// A segment in registers: its |x|max bits (fp32 bits for fp32 input, bf16 bits
+// for bf16), and, where the hint admits the instruction path, its codes at
+// the hinted exponent.
 template <int FMT, bool BF16>
-__global__ __launch_bounds__(kQBlock) void quant_hint_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
-                                                             int32_t k_hint, const int32_t* k_hint_dev,
-                                                             int32_t hint_is_amax, uint8_t* __restrict__ q,
-                                                             void* __restrict__ out, uint32_t* __restrict__ partial,
-                                                             int32_t* __restrict__ hint_copy) {
-    constexpr int VPL = Seg<BF16>::VPL;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t seg = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
-    if (seg >= segs) return;
-    int32_t hint = k_hint;
-    if (k_hint_dev) {
-        hint = __builtin_amdgcn_readfirstlane(*k_hint_dev);
-        if (hint_is_amax) hint = scale_exp_from_amax<FMT>((uint32_t)hint);
-    }
-    if (seg == 0 && lane == 0) hint_copy[0] = hint;
+__device__ __forceinline__ uint32_t hint_segment(const uint4 (&buf)[Seg<BF16>::VPL], const SegAt<BF16>& at, int32_t hint,
+                                                 uint8_t* q, void* out, int lane) {
     const bool convert = hint >= -kFastK && hint <= kFastK;
     RowScale hs;
     hs.k = hint;
     hs.fast = true;
     hs.s_down = __uint_as_float((uint32_t)(127 - hint) << 23);
     hs.s_up = __uint_as_float((uint32_t)(127 + hint) << 23);
-    uint4 buf[VPL];
-    const SegAt<BF16> at(seg, n);
-    load_segment<BF16>(static_cast<const char*>(x), at, lane, buf);
     uint32_t amax = 0;
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) {
+    for (int j = 0; j < Seg<BF16>::VPL; ++j) {
         amax = vec_absmax<BF16>(buf[j], amax);
         if (convert) convert_seg_vec<FMT, BF16>(buf[j], at, lane + kWave * j, 0, hs, q, out);
     }
-    amax = wave_max_u32(amax);
+    return wave_max_u32(amax);
+}
+
+// The hint: k_hint, or *k_hint_dev when that is given (read here, before
+// the fixup launch writes k, which may be the same word).  Wave 0 keeps the
+// hint it read in hint_copy for the fixup.  A hint outside the instruction
+// path's range converts nothing here: the call is then a miss.
+template <int FMT, bool BF16>
+__global__ __launch_bounds__(kQBlock) void quant_hint_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
+                                                             int32_t k_hint, const int32_t* k_hint_dev,
+                                                             uint8_t* __restrict__ q, void* __restrict__ out,
+                                                             uint32_t* __restrict__ partial,
+                                                             int32_t* __restrict__ hint_copy) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t seg = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
+    if (seg >= segs) return;
+    const int32_t hint = k_hint_dev ? __builtin_amdgcn_readfirstlane(*k_hint_dev) : k_hint;
+    if (seg == 0 && lane == 0) hint_copy[0] = hint;
+    const SegAt<BF16> at(seg, n);
+    uint4 buf[Seg<BF16>::VPL];
+    load_segment<BF16>(static_cast<const char*>(x), at, lane, buf);
+    const uint32_t amax = hint_segment<FMT, BF16>(buf, at, hint, q, out, lane);
     if (lane == 0) partial[seg] = amax;
 }
 
-// A per-tensor row's exponent guessed from a sample: wave w reads segment
-// w * stride (stride a prime, so that the sample does not fall in step with
-// a row length or an outlier channel) and writes its |x|max, as fp32 bits,
-// to partial[w].  The vector form only (n a whole number of 16-byte
-// vectors, aligned x).
+// A per-tensor row's exponent guessed from a sample, in three launches:
+//   * guess_amax_kernel: kGuessBlocks blocks fold the |x|max of every
+//     kGuessStride-th segment (a prime, so that the sample does not fall in
+//     step with a row length or an outlier channel) to one word each, and
+//     clear the tops;
+//   * quant_guess_kernel: every wave folds those words to the sample's |x|max
+//     while its segment is on the way, converts at its exponent, and raises
+//     a top where its segment exceeds the sample (none to a few dozen
+//     segments of a tensor whose values come in no order; at worst, every
+//     segment of a rising one, spread over kTops words, a line each);
+//   * the fixup folds the sample and the tops to the row's |x|max: it exits
+//     where that has the guessed exponent, and converts again where not.
+// All |x|max words here are fp32 bits.  Against five launches (the sample's
+// words folded by one, the segments' maxima of the hint path by another),
+// bf16, right guesses: 64 MiB 29.4 -> 24.0 us, 128 MiB 45.1 -> 38.8, 1 GiB
+// 265 -> 253 (6.37 TB/s).  A miss with every unsampled segment above the
+// sample (most atomics): 128 MiB 72.7 -> 66.3 us, 1 GiB 530 -> 515.
+constexpr int kGuessBlocks = 256, kGuessBlockWaves = 8;
+constexpr int kTops = 64, kTopStride = 32;  // words: a top per lane of a fixup wave, 128 bytes apart
 template <bool BF16>
-__global__ __launch_bounds__(kQBlock) void guess_amax_kernel(const void* __restrict__ x, int64_t n, int64_t stride,
-                                                             int64_t samples, uint32_t* __restrict__ partial) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t w = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
-    if (w >= samples) return;
-    const uint32_t m = wave_max_u32(seg_absmax<BF16, (ELY_FP8_NT & 1) != 0>(x, 0, n, w * stride, 1, lane));
-    if (lane == 0) partial[w] = to_f32_bits<BF16>(m);
-}
-
-// out[0] = max of partial[0, count): one block (an integer max, order-free;
-// one word per sample, so no same-address atomics serialize the guess).
-constexpr int kSampleMaxBlock = 1024;
-__global__ __launch_bounds__(kSampleMaxBlock) void sample_max_kernel(const uint32_t* __restrict__ partial,
-                                                                    int64_t count, uint32_t* __restrict__ out) {
-    __shared__ uint32_t red[kSampleMaxBlock / kWave];
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+__global__ __launch_bounds__(kGuessBlockWaves * kWave) void guess_amax_kernel(const void* __restrict__ x, int64_t n,
+                                                                              int64_t stride, int64_t samples,
+                                                                              uint32_t* __restrict__ sampled,
+                                                                              uint32_t* __restrict__ tops) {
+    __shared__ uint32_t red[kGuessBlockWaves];
+    const int lane = threadIdx.x & (kWave - 1), w = wave_uniform(threadIdx.x / kWave);
     uint32_t m = 0;
-#pragma unroll 4
-    for (int64_t i = threadIdx.x; i < count; i += kSampleMaxBlock) m = max(m, partial[i]);
+    for (int64_t i = blockIdx.x + (int64_t)w * kGuessBlocks; i < samples; i += kGuessBlocks * kGuessBlockWaves)
+        m = max(m, seg_absmax<BF16, (ELY_FP8_NT & 1) != 0>(x, 0, n, i * stride, 1, lane));
     m = wave_max_u32(m);
     if (lane == 0) red[w] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t r = red[0];
-        for (int j = 1; j < kSampleMaxBlock / kWave; ++j) r = max(r, red[j]);
-        out[0] = r;
+#pragma unroll
+        for (int i = 1; i < kGuessBlockWaves; ++i) m = max(m, red[i]);
+        sampled[blockIdx.x] = to_f32_bits<BF16>(m);
+        if (blockIdx.x < kTops) tops[blockIdx.x * kTopStride] = 0;
     }
+}
+
+template <int FMT, bool BF16>
+__global__ __launch_bounds__(kQBlock) void quant_guess_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
+                                                              const uint32_t* __restrict__ sampled,
+                                                              uint8_t* __restrict__ q, void* __restrict__ out,
+                                                              uint32_t* __restrict__ tops, uint32_t* __restrict__ amax) {
+    static_assert(kGuessBlocks == 4 * kWave, "a lane folds four sampled words");
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t seg = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
+    if (seg >= segs) return;
+    const SegAt<BF16> at(seg, n);
+    uint4 buf[Seg<BF16>::VPL];
+    load_segment<BF16>(static_cast<const char*>(x), at, lane, buf);
+    const uint32_t sample = __builtin_amdgcn_readfirstlane(wave_max_u32(
+        max(max(sampled[lane], sampled[lane + kWave]), max(sampled[lane + 2 * kWave], sampled[lane + 3 * kWave]))));
+    if (seg == 0 && lane == 0) amax[0] = sample;
+    const uint32_t top = to_f32_bits<BF16>(hint_segment<FMT, BF16>(buf, at, scale_exp_from_amax<FMT>(sample), q, out, lane));
+    if (lane == 0 && top > sample) atomicMax(tops + (seg % kTops) * kTopStride, top);
 }
 
 // partial[0, segs) -> out[b] for b < kHintBlocks (block b folds a contiguous
@@ -754,27 +778,47 @@ __global__ __launch_bounds__(kRowBlock) void hint_reduce_kernel(const uint32_t* 
     }
 }
 
+// The fixup of a hinted or guessed row whose |x|max bits are m: k and the hit
+// flag, and, on a miss, every segment again at the true scale.
 template <int FMT, bool BF16>
-__global__ __launch_bounds__(kQBlock) void quant_hint_fixup_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
-                                                                   int vec, const int32_t* __restrict__ hint_copy,
-                                                                   const uint32_t* __restrict__ block_max,
-                                                                   uint8_t* __restrict__ q, int32_t* __restrict__ k,
-                                                                   void* __restrict__ out, int32_t* __restrict__ hit) {
-    static_assert(kHintBlocks == 4 * kWave, "a fixup lane folds four block maxima");
-    const int lane = threadIdx.x & (kWave - 1);
+__device__ __forceinline__ void fixup(const void* x, int64_t n, int64_t segs, int32_t hint, uint32_t m, uint8_t* q, int32_t* k,
+                                      void* out, int32_t* hit, int lane) {
     const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave_uniform(threadIdx.x / kWave);
     const int64_t waves = (int64_t)gridDim.x * kWavesPerBlock;
-    uint32_t m = max(max(block_max[lane], block_max[lane + kWave]), max(block_max[lane + 2 * kWave], block_max[lane + 3 * kWave]));
-    m = wave_max_u32(m);
-    const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(m), BF16, BF16);
-    const int32_t k_hint = hint_copy[0];
-    const bool same = rs.fast && rs.k == k_hint && k_hint >= -kFastK && k_hint <= kFastK;
+    const RowScale rs = row_scale<FMT>(m, BF16, BF16);
+    const bool same = rs.fast && rs.k == hint && hint >= -kFastK && hint <= kFastK;
     if (gw == 0 && lane == 0) {
         k[0] = rs.k;
         if (hit) hit[0] = same ? 1 : 0;
     }
     if (same) return;
-    for (int64_t seg = gw; seg < segs; seg += waves) quant_segment<FMT, BF16>(x, 0, n, seg, vec, rs, q, out, lane);
+    for (int64_t seg = gw; seg < segs; seg += waves) quant_segment<FMT, BF16>(x, 0, n, seg, 1, rs, q, out, lane);
+}
+
+template <int FMT, bool BF16>
+__global__ __launch_bounds__(kQBlock) void quant_hint_fixup_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
+                                                                   const int32_t* __restrict__ hint_copy,
+                                                                   const uint32_t* __restrict__ block_max,
+                                                                   uint8_t* __restrict__ q, int32_t* __restrict__ k,
+                                                                   void* __restrict__ out, int32_t* __restrict__ hit) {
+    static_assert(kHintBlocks == 4 * kWave, "a fixup lane folds four block maxima");
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t m = wave_max_u32(max(max(block_max[lane], block_max[lane + kWave]),
+                                        max(block_max[lane + 2 * kWave], block_max[lane + 3 * kWave])));
+    fixup<FMT, BF16>(x, n, segs, hint_copy[0], to_f32_bits<BF16>(m), q, k, out, hit, lane);
+}
+
+template <int FMT, bool BF16>
+__global__ __launch_bounds__(kQBlock) void quant_guess_fixup_kernel(const void* __restrict__ x, int64_t n, int64_t segs,
+                                                                    const uint32_t* __restrict__ tops,
+                                                                    const uint32_t* __restrict__ amax,
+                                                                    uint8_t* __restrict__ q, int32_t* __restrict__ k,
+                                                                    void* __restrict__ out) {
+    static_assert(kTops == kWave, "a fixup lane reads one top");
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t sample = amax[0];
+    const uint32_t m = wave_max_u32(max(sample, tops[lane * kTopStride]));
+    fixup<FMT, BF16>(x, n, segs, scale_exp_from_amax<FMT>(sample), m, q, k, out, nullptr, lane);
 }
 
 // -------------------------------------------------------------- dequantize
@@ -1581,14 +1625,12 @@ static size_t hint_ws_bytes(int64_t n) {
 template <int FMT, bool BF16>
 static void quantize_hint_impl(const void* x, int64_t n, int32_t k_hint, const int32_t* k_hint_dev, uint8_t* q,
                                int32_t* k, void* out, int32_t* hit, void* workspace, int64_t ws_bytes,
-                               hipStream_t s, bool hint_is_amax = false) {
+                               hipStream_t s) {
     if (!workspace || ws_bytes < (int64_t)hint_ws_bytes(n))
         fail(ELY_EWORKSPACE, "ely_fp8_quantize_hint: workspace of " + std::to_string(ws_bytes) + " bytes, need " +
                                  std::to_string(hint_ws_bytes(n)) + " (ely_fp8_hint_workspace_bytes)");
-    // a caller's hint keeps to whole aligned vectors (*hit says so); a guess
-    // takes any row of at least one
-    const int32_t dt = BF16 ? ELY_BF16 : ELY_F32;
-    const bool vec = n > 0 && (hint_is_amax ? any_vecs(n, dt, x, out) : whole_vecs(n, dt, x, q, out));
+    // the one-pass form keeps to whole aligned vectors (*hit says so)
+    const bool vec = n > 0 && whole_vecs(n, BF16 ? ELY_BF16 : ELY_F32, x, q, out);
     if (!vec || (!k_hint_dev && (k_hint < -kFastK || k_hint > kFastK))) {
         // no one-pass form for this tensor or hint: the split path, a miss
         quantize_impl<FMT, BF16>(x, 1, n, q, k, out, workspace, ws_bytes, s, false);
@@ -1603,45 +1645,49 @@ static void quantize_hint_impl(const void* x, int64_t n, int32_t k_hint, const i
     uint32_t* block_max = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + align_up((size_t)segs * 4, 256));
     int32_t* hint_copy = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(block_max) + align_up((size_t)kHintBlocks * 4, 256));
     hipLaunchKernelGGL((quant_hint_kernel<FMT, BF16>), dim3(blocks_for_waves(segs)), dim3(kQBlock), 0, s, x, n, segs,
-                       k_hint, k_hint_dev, hint_is_amax ? 1 : 0, q, out, partial, hint_copy);
+                       k_hint, k_hint_dev, q, out, partial, hint_copy);
     check_launch("quant_hint_kernel");
     hipLaunchKernelGGL(hint_reduce_kernel, dim3(kHintBlocks), dim3(kRowBlock), 0, s, (const uint32_t*)partial, segs,
                        block_max);
     check_launch("hint_reduce_kernel");
     const int64_t waves = std::min<int64_t>(segs, (int64_t)device_info().cus * kHintFixupWavesPerCU);
     hipLaunchKernelGGL((quant_hint_fixup_kernel<FMT, BF16>), dim3(blocks_for_waves(waves)), dim3(kQBlock), 0, s, x, n,
-                       segs, 1, (const int32_t*)hint_copy, (const uint32_t*)block_max, q, k, out, hit);
+                       segs, (const int32_t*)hint_copy, (const uint32_t*)block_max, q, k, out, hit);
     check_launch("quant_hint_fixup_kernel");
 }
 
 // Per-tensor rows of at least ELY_GUESS_MIN_MB MiB (the vector form, a
 // workspace of guess_ws_bytes): the exponent is guessed from every
-// kGuessStride-th segment's |x|max, and the row goes through the hint path
-// at that guess: one read of x when the sample holds the row's maximum
-// binade, the hint path's fixup (a second read and write) when it does not.
-// Either way the codes and k are the split path's, byte for byte.  C4
-// per-tensor (both inputs guess right), kernel time per call: quantize
-// 272 us against 404 on the split path, round trip 357 against 488.
+// kGuessStride-th segment's |x|max, and the row is converted at that guess:
+// one read of x when the sample holds the row's maximum binade, the fixup (a
+// second read and write) when it does not.  Either way the codes and k are
+// the split path's, byte for byte.
 static size_t guess_ws_bytes(int64_t n) { return hint_ws_bytes(n) + 256; }
+static_assert(((int64_t)ELY_GUESS_MIN_MB << 20) / 4 / kSegElems >= kGuessBlocks + kTops * kTopStride,
+              "the shortest guessed row's workspace holds the sampled words and the tops");
 
 template <int FMT, bool BF16>
 static void quantize_guess_impl(const void* x, int64_t n, uint8_t* q, int32_t* k, void* out, void* workspace,
                                 int64_t ws_bytes, hipStream_t s) {
     // after the hint path's layout: the sampled |x|max, and k's word when
-    // the caller asked for no k (a round trip); the samples' maxima go where
-    // the hint path's per-segment maxima go later (samples <= segments)
+    // the caller asked for no k (a round trip); the sampled words and the tops
+    // take the first bytes of what the hint path keeps its maxima in
     uint32_t* amax = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + hint_ws_bytes(n));
     int32_t* kword = k ? k : reinterpret_cast<int32_t*>(amax + 1);
-    uint32_t* partial = static_cast<uint32_t*>(workspace);
+    uint32_t* sampled = static_cast<uint32_t*>(workspace);
+    uint32_t* tops = sampled + kGuessBlocks;
     const int64_t segs = (n + kSegElems - 1) / kSegElems;
     const int64_t samples = (segs + kGuessStride - 1) / kGuessStride;
-    hipLaunchKernelGGL((guess_amax_kernel<BF16>), dim3(blocks_for_waves(samples)), dim3(kQBlock), 0, s, x, n,
-                       (int64_t)kGuessStride, samples, partial);
+    hipLaunchKernelGGL((guess_amax_kernel<BF16>), dim3(kGuessBlocks), dim3(kGuessBlockWaves * kWave), 0, s, x, n,
+                       (int64_t)kGuessStride, samples, sampled, tops);
     check_launch("guess_amax_kernel");
-    hipLaunchKernelGGL(sample_max_kernel, dim3(1), dim3(kSampleMaxBlock), 0, s, (const uint32_t*)partial, samples, amax);
-    check_launch("sample_max_kernel");
-    quantize_hint_impl<FMT, BF16>(x, n, 0, reinterpret_cast<const int32_t*>(amax), q, kword, out, nullptr, workspace,
-                                  ws_bytes, s, true);
+    hipLaunchKernelGGL((quant_guess_kernel<FMT, BF16>), dim3(blocks_for_waves(segs)), dim3(kQBlock), 0, s, x, n, segs,
+                       (const uint32_t*)sampled, q, out, tops, amax);
+    check_launch("quant_guess_kernel");
+    const int64_t waves = std::min<int64_t>(segs, (int64_t)device_info().cus * kHintFixupWavesPerCU);
+    hipLaunchKernelGGL((quant_guess_fixup_kernel<FMT, BF16>), dim3(blocks_for_waves(waves)), dim3(kQBlock), 0, s, x, n,
+                       segs, (const uint32_t*)tops, (const uint32_t*)amax, q, kword, out);
+    check_launch("quant_guess_fixup_kernel");
 }
 
 template <int FMT, bool BF16OUT, bool RAGGED>

@@ -96,8 +96,11 @@ def test_a_ragged_tensor_past_the_guess_size_equals_torch(off):
     n = (1 << 25) + 2048 + 5
     g = torch.Generator(device="cuda").manual_seed(off)
     x = torch.randn(n + off, generator=g, device="cuda").bfloat16()[off:]
-    for top in (None, 1e4):
-        if top is not None:
+    for top in (None, 1e4, "rising"):
+        if top == "rising":  # every segment that the guess does not sample exceeds those it does
+            x[: n // 2048 * 2048].view(-1, 2048)[::61] *= 2.0**-5
+            x[n - 2] = 0.25
+        elif top is not None:
             x[n - 2] = top
         say("fp8 ragged guess", off, top)
         q, k = fp8.quantize(x, "e4m3", per_tensor=True)
