@@ -9,16 +9,12 @@ both carrying ely_last_error().
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 import threading
 
 import numpy as np
 import torch
-
-try:
-    from . import _native
-except ImportError as e:  # not built yet: load_native() says so at the first call
-    _native, _native_error = None, e
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libelyhip.so")
@@ -146,14 +142,39 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return _lib
 
 
+class _Unbuilt:
+    """Stands for _native where nothing has been built: every plain call is
+    declined, so that the Python code behind it answers what needs no library
+    and says of the rest that the library is missing."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+    def workspace(self, index, nbytes):
+        load()  # raises
+
+
+_native = None
+_unbuilt = _Unbuilt()
+
+
 def load_native():
-    """The module of the plain calls (csrc/binding.cpp); raises RuntimeError
-    when it has not been built."""
-    if _native is None:
+    """The module of the plain calls (csrc/binding.cpp), loaded at the first
+    call: importing the package maps no library, so that one built after the
+    import is the one that runs."""
+    global _native
+    if _native is not None:
+        return _native
+    if not os.path.exists(LIB_PATH):
+        return _unbuilt
+    importlib.invalidate_caches()  # it may have been built since the last look
+    try:
+        _native = importlib.import_module("._native", __package__)
+    except ImportError as e:
         raise RuntimeError(
-            f"elysium_wan_amd._native cannot be loaded ({_native_error}): build the HIP library first "
+            f"elysium_wan_amd._native cannot be loaded ({e}): build the HIP library first "
             "(python -m elysium_wan_amd.build, or __graft_entry__.build())"
-        )
+        ) from e
     return _native
 
 

@@ -3,10 +3,20 @@ any effect, so that the Python code behind them answers as it always did."""
 
 from __future__ import annotations
 
+import glob
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
+from conftest import ROOT
 from elysium_wan_amd import _lib
+
+PACKAGE = os.path.join(ROOT, "elysium_wan_amd")
+LIBRARIES = ("libelyhip.so", "_native.so")
 
 
 class _Sub(torch.Tensor):
@@ -25,6 +35,68 @@ def test_host_tensors_and_other_objects_are_declined():
     p = torch.zeros(4)
     args = [[p], [torch.ones(4)], None, {}, torch.zeros(1), None, 0, 0, 0, None, None, lambda t: [0.0] * 8]
     assert _lib.load_native().adamw_step(*args) is None and float(args[4][0]) == 0.0
+
+
+def _copy_of_the_package(tmp_path, *names):
+    d = tmp_path / "elysium_wan_amd"
+    d.mkdir()
+    for f in glob.glob(os.path.join(PACKAGE, "*.py")) + [os.path.join(PACKAGE, n) for n in names]:
+        shutil.copy(f, d)
+    return d
+
+
+def _run(tmp_path, code):
+    r = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True, timeout=120,
+                       env={**os.environ, "PYTHONDONTWRITEBYTECODE": "1"})
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_a_library_built_after_the_import_is_used(tmp_path):
+    """Nothing built: host calls answer as they do with the libraries, the
+    rest say what is missing; once the libraries are there, they load."""
+    _copy_of_the_package(tmp_path)
+    _run(tmp_path, f"""
+import shutil, torch
+from elysium_wan_amd import _lib, fp8, optim, pieces
+
+n = torch.tensor([3])
+pieces.fold_add(n, torch.tensor([4]))
+assert int(n) == 7 and float(optim.clip_grad_norm_([torch.zeros(2)], 1.0)) == 0.0
+for call, error in ((lambda: fp8.quantize(torch.zeros(2, 8)), ValueError), (lambda: pieces.cast_piece(torch.zeros(8), torch.bfloat16), ValueError),
+                    (lambda: _lib.workspace(torch.device("cuda", 0), 1), RuntimeError), (lambda: _lib.load(), RuntimeError)):
+    try:
+        call()
+    except error as e:
+        assert "GPU" in str(e) or "build the HIP library" in str(e), e
+    else:
+        raise AssertionError("not refused")
+shutil.copy({os.path.join(PACKAGE, LIBRARIES[0])!r}, "elysium_wan_amd")
+try:
+    _lib.load_native()
+except RuntimeError as e:
+    assert "build the HIP library" in str(e), e
+else:
+    raise AssertionError("loaded without its file")
+shutil.copy({os.path.join(PACKAGE, LIBRARIES[1])!r}, "elysium_wan_amd")
+assert _lib.load_native().quantize(torch.zeros(2, 8), "e4m3", False) is None and _lib.load().ely_abi_version() == 1
+""")
+
+
+def test_a_library_rebuilt_after_the_import_is_the_one_that_runs(tmp_path):
+    _copy_of_the_package(tmp_path, *LIBRARIES)
+    _run(tmp_path, """
+import os, shutil
+import elysium_wan_amd
+from elysium_wan_amd import _lib, accumulate, boundary, f32_planes, fp8, fp8_planes, optim, pieces, planes
+
+for name in ("libelyhip.so", "_native.so"):
+    shutil.copy("elysium_wan_amd/" + name, "new")
+    os.replace("new", "elysium_wan_amd/" + name)
+_lib.load(), _lib.load_native()
+for name in ("libelyhip.so", "_native.so"):
+    mapped = {line.split()[4] for line in open("/proc/self/maps") if "/elysium_wan_amd/" + name in line}
+    assert mapped == {str(os.stat("elysium_wan_amd/" + name).st_ino)}, (name, mapped)
+""")
 
 
 @pytest.mark.gpu
