@@ -9,13 +9,13 @@
 //   acc[idx[j]] += a[rows_a[j]] + 0.0                  (later, free rows)
 //   acc[idx[j]]  = a[j] + e_j       / acc[idx[j]] += a[j] + e_j
 //                                                      (held rows resolved)
-// over a set of distinct rows, which this kernel runs: a wave per piece of a
-// row, 16-byte vectors across it.  e_j is the
-// embedding row b[b_rows[j]] of a held row the microbatch touched, +0.0 for
+// over a set of distinct rows, which this kernel runs: a block per row or
+// piece of a row, 16-byte vectors across it.  e_j is the embedding row b[b_rows[j]] of a held row the microbatch touched, +0.0 for
 // one it did not (b_rows[j] < 0), or b[j] of a compact b.  A second kernel
 // takes a whole Head gradient in one pass: its free rows fold, its held
 // rows are copied out bit for bit, so that the gradient itself can go.
 #include <algorithm>
+#include <type_traits>
 
 #include "ely_device.hpp"
 #include "ely_host.hpp"
@@ -25,16 +25,16 @@
 namespace ely {
 namespace {
 
-// A wave moves V 16-byte vectors per lane of a row and ends, a row's pieces
-// across the grid, rows down (a longer list strides).  Launches that touch
-// more than the 256 MB MALL holds stream (nontemporal loads, and the split's
-// stores); the others keep to plain loads, for the rows and the sum are read
-// again soon.  Against a 256-thread block per row, in one process on the same
-// buffers, a third of the rows held: 32,768 x 2,560 fp32 split 170 -> 142 us
-// (5.3 -> 6.3 TB/s) and fold of the held 77 -> 61, bf16 84 -> 74 and 32 -> 32,
-// 8,192 x 1,024 fp32 14.4 both and 7.0 -> 7.6; 32,768 x 1,001 bf16, element
-// by element before, 89 -> 40 and 27 -> 17.
-constexpr int kSplitVecs = 2, kFoldVecs = 1;
+// A block of W waves moves V 16-byte vectors per lane of a row and ends, a
+// row's pieces across the grid, rows down (a longer list strides).  Launches
+// that touch more than the 256 MB MALL holds stream (nontemporal loads, and
+// the split's stores), one-wave blocks taking the pieces; the others keep to
+// plain accesses, for the rows and the sum are read again soon, in the shapes
+// of fold_shape and split_shape.  Streaming, against a 256-thread block that
+// loops over its row, buffers in turn, a third of the rows held: 32,768 x
+// 2,560 fp32 split 166 -> 146 us (5.1 -> 5.8 TB/s) and fold of the held 77 ->
+// 60, bf16 84 -> 76 and 40 -> 40; 32,768 x 1,001 bf16, element by element
+// before, 90 -> 43 and 40 -> 21.
 constexpr int64_t kMallBytes = (int64_t)256 << 20;
 constexpr int64_t kRowGrid = 65535;
 
@@ -86,16 +86,16 @@ __device__ __forceinline__ ru4 fold_vec(ru4 z, ru4 x, ru4 y, int first) {
 // Piece `piece` of one row of d elements: ac (=|+=) av + (bv or +0.0), its
 // vectors' loads all issued before the first is stored.  The row's last
 // elements, short of a vector, go to the last piece's lanes, one each.
-template <bool BF16, int V, bool NTL, bool NTS>
+template <bool BF16, int V, int W, bool NTL, bool NTS>
 __device__ __forceinline__ void fold_piece(char* ac, const char* av, const char* bv, int64_t d, int piece, int first,
                                            int vec) {
-    constexpr int EPV = BF16 ? 8 : 4, ESZ = BF16 ? 2 : 4;
+    constexpr int EPV = BF16 ? 8 : 4, T = kWave * W;
     const int64_t nvec = vec ? d / EPV : 0;
-    const int64_t v0 = (int64_t)piece * (kWave * V) + threadIdx.x;
+    const int64_t v0 = (int64_t)piece * (T * V) + threadIdx.x;
     ru4 x[V], y[V], z[V];
 #pragma unroll
     for (int u = 0; u < V; ++u) {
-        const int64_t v = v0 + u * kWave;
+        const int64_t v = v0 + u * T;
         const ru4 zero = {0u, 0u, 0u, 0u};
         x[u] = v < nvec ? ld_row<NTL>(av + v * 16) : zero;
         y[u] = (v < nvec && bv) ? ld_row<NTL>(bv + v * 16) : zero;
@@ -103,11 +103,11 @@ __device__ __forceinline__ void fold_piece(char* ac, const char* av, const char*
     }
 #pragma unroll
     for (int u = 0; u < V; ++u) {
-        const int64_t v = v0 + u * kWave;
+        const int64_t v = v0 + u * T;
         if (v < nvec) st_row<NTS>(ac + v * 16, fold_vec<BF16>(z[u], x[u], y[u], first));
     }
     if (piece != (int)gridDim.x - 1) return;
-    for (int64_t c = nvec * EPV + threadIdx.x; c < d; c += kWave) {
+    for (int64_t c = nvec * EPV + threadIdx.x; c < d; c += T) {
         if (BF16) {
             uint16_t* o = reinterpret_cast<uint16_t*>(ac) + c;
             const float z1 = first ? 0.0f : bf16_to_f32(*o);
@@ -121,14 +121,14 @@ __device__ __forceinline__ void fold_piece(char* ac, const char* av, const char*
     }
 }
 
-template <bool BF16, bool NT>
-__global__ __launch_bounds__(kWave) void rows_fold_kernel(void* __restrict__ acc, const void* __restrict__ a,
-                                                          const int64_t* __restrict__ a_rows,
-                                                          const void* __restrict__ b,
-                                                          const int64_t* __restrict__ b_rows,
-                                                          const int64_t* __restrict__ idx, int64_t n_idx,
-                                                          int64_t n_rows, int64_t a_total, int64_t b_total,
-                                                          int64_t d, int first, int vec) {
+template <bool BF16, int V, int W, bool NT>
+__global__ __launch_bounds__(kWave * W) void rows_fold_kernel(void* __restrict__ acc, const void* __restrict__ a,
+                                                              const int64_t* __restrict__ a_rows,
+                                                              const void* __restrict__ b,
+                                                              const int64_t* __restrict__ b_rows,
+                                                              const int64_t* __restrict__ idx, int64_t n_idx,
+                                                              int64_t n_rows, int64_t a_total, int64_t b_total,
+                                                              int64_t d, int first, int vec) {
     const int64_t esz = BF16 ? 2 : 4;
     for (int64_t j = blockIdx.y; j < n_idx; j += gridDim.y) {
         const int64_t r = idx[j];
@@ -136,28 +136,27 @@ __global__ __launch_bounds__(kWave) void rows_fold_kernel(void* __restrict__ acc
         const int64_t br = b ? (b_rows ? b_rows[j] : j) : -1;  // < 0: the row adds +0.0
         // the host checks every index; a row outside the tables is skipped, never touched
         if (r < 0 || r >= n_rows || ar < 0 || ar >= a_total || br >= b_total) continue;
-        fold_piece<BF16, kFoldVecs, NT, false>(static_cast<char*>(acc) + r * d * esz,
-                                               static_cast<const char*>(a) + ar * d * esz,
-                                               br >= 0 ? static_cast<const char*>(b) + br * d * esz : nullptr, d,
-                                               blockIdx.x, first, vec);
+        fold_piece<BF16, V, W, NT, false>(static_cast<char*>(acc) + r * d * esz, static_cast<const char*>(a) + ar * d * esz,
+                                          br >= 0 ? static_cast<const char*>(b) + br * d * esz : nullptr, d, blockIdx.x,
+                                          first, vec);
     }
 }
 
 // That piece of a row of d elements copied bit for bit.
-template <bool BF16, int V, bool NTL>
+template <bool BF16, int V, int W, bool NT>
 __device__ __forceinline__ void copy_piece(char* o, const char* x, int64_t d, int piece, int vec) {
-    constexpr int EPV = BF16 ? 8 : 4, ESZ = BF16 ? 2 : 4;
+    constexpr int EPV = BF16 ? 8 : 4, ESZ = BF16 ? 2 : 4, T = kWave * W;
     const int64_t nvec = vec ? d / EPV : 0;
-    const int64_t v0 = (int64_t)piece * (kWave * V) + threadIdx.x;
+    const int64_t v0 = (int64_t)piece * (T * V) + threadIdx.x;
     ru4 t[V];
 #pragma unroll
     for (int u = 0; u < V; ++u)
-        if (v0 + u * kWave < nvec) t[u] = ld_row<NTL>(x + (v0 + u * kWave) * 16);
+        if (v0 + u * T < nvec) t[u] = ld_row<NT>(x + (v0 + u * T) * 16);
 #pragma unroll
     for (int u = 0; u < V; ++u)
-        if (v0 + u * kWave < nvec) st_row<true>(o + (v0 + u * kWave) * 16, t[u]);
+        if (v0 + u * T < nvec) st_row<NT>(o + (v0 + u * T) * 16, t[u]);
     if (piece != (int)gridDim.x - 1) return;
-    for (int64_t c = nvec * 16 + threadIdx.x; c < d * ESZ; c += kWave) o[c] = x[c];
+    for (int64_t c = nvec * 16 + threadIdx.x; c < d * ESZ; c += T) o[c] = x[c];
 }
 
 // A Head gradient in one pass, a row's pieces across the grid: a row r with
@@ -165,8 +164,8 @@ __device__ __forceinline__ void copy_piece(char* o, const char* x, int64_t d, in
 // acc[r] + (a[r] + 0.0), each add rounded to the dtype; a held row
 // (slot[r] >= 0) is copied to held_out[slot[r]] bit for bit and acc[r] is
 // left for its resolve.
-template <bool BF16, bool NT>
-__global__ __launch_bounds__(kWave) void rows_split_kernel(void* __restrict__ acc, const void* __restrict__ a,
+template <bool BF16, int V, int W, bool NT>
+__global__ __launch_bounds__(kWave * W) void rows_split_kernel(void* __restrict__ acc, const void* __restrict__ a,
                                                                const int32_t* __restrict__ slot,
                                                                void* __restrict__ held_out, int64_t n_rows,
                                                                int64_t n_held, int64_t d, int first, int vec) {
@@ -175,22 +174,66 @@ __global__ __launch_bounds__(kWave) void rows_split_kernel(void* __restrict__ ac
         const int64_t s = slot[r];
         const char* x = static_cast<const char*>(a) + r * row_bytes;
         if (s < 0)
-            fold_piece<BF16, kSplitVecs, NT, true>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, blockIdx.x, first, vec);
+            fold_piece<BF16, V, W, NT, NT>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, blockIdx.x, first, vec);
         else if (s < n_held)  // the host numbers the held rows 0..n_held-1
-            copy_piece<BF16, kSplitVecs, NT>(static_cast<char*>(held_out) + s * row_bytes, x, d, blockIdx.x, vec);
+            copy_piece<BF16, V, W, NT>(static_cast<char*>(held_out) + s * row_bytes, x, d, blockIdx.x, vec);
     }
 }
 
-// The pieces of a row of d elements across, rows down; a dispatch counts its
-// threads in 32 bits.
-dim3 rows_grid(int64_t rows, int64_t d, int64_t esz, int vec, int vecs, const char* what) {
-    const int64_t per = (int64_t)kWave * vecs;
-    const int64_t pieces = vec ? std::max<int64_t>(1, (d * esz / 16 + per - 1) / per) : 1;
-    if (pieces > 0xFFFFFFFFLL / kWave) fail(ELY_EINVAL, std::string(what) + ": rows too long for one launch");
-    return dim3((unsigned)pieces, (unsigned)std::min({rows, kRowGrid, (int64_t)0xFFFFFFFFLL / (kWave * pieces)}));
+// The pieces of a row (`span` vectors a block) across, rows down, for blocks
+// of `threads`; a dispatch counts its threads in 32 bits.
+dim3 rows_grid(int64_t rows, int64_t nvec, int64_t span, int64_t threads) {
+    const int64_t pieces = std::max<int64_t>(1, (nvec + span - 1) / span);
+    return dim3((unsigned)pieces, (unsigned)std::min({rows, kRowGrid, (int64_t)0xFFFFFFFFLL / (threads * pieces)}));
 }
 
+// The shapes of launches that do not stream, by a row's vectors.  A block that
+// holds its whole row is the fastest where the lanes it leaves idle are few: 1,
+// 2 and 4 waves of a vector a lane up to 64, 128 and 256 vectors, 4 waves of two
+// up to 512.  (A row of two blocks, the second nearly empty, puts the empty
+// ones on every second XCD: 320 vectors 12.4 us against 9.8 in one-wave
+// pieces.)  Past 512 a row is cut in pieces again.  The fold of few rows, and
+// of long bf16 rows, is the faster on one-wave pieces; so is the split of more
+// than 32 MB of bf16, two vectors a lane.
+// The launches of four microbatches (split and fold each), from a graph, in us,
+// with a looping 256-thread block per row / one-wave pieces at every size /
+// these: fp32 256 x 1,024 17.1 / 18.4 / 16.5, 4,096 x 768 41.8 / 46.9 / 41.9,
+// 8,192 x 1,024 82 / 87 / 81, 16,384 x 1,600 230 / 252 / 235; bf16 256 x 768
+// 19.6 / 22.5 / 19.2, 8,192 x 2,048 88 / 95 / 89, 32,768 x 768 179 / 140 / 138.
+// One by one, a third of 8,192 x 1,024 fp32 rows folded again and again: 5.7 /
+// 7.8 / 5.5; 16,384 x 1,600 split 42.5 / 49.0 / 42.0.
+struct RowShape {
+    int v, w;
+};
+RowShape fold_shape(int64_t rows, int64_t nvec, bool bf16) {
+    if (rows <= 512 || nvec <= kWave || (bf16 && nvec > 4 * kWave)) return {1, 1};
+    if (nvec <= 2 * kWave) return {1, 2};
+    if (nvec <= 4 * kWave) return {1, 4};
+    if (nvec <= 7 * kWave) return {2, 4};
+    if (nvec <= 8 * kWave) return {1, 4};
+    if (nvec <= 12 * kWave) return {2, 2};
+    return {1, 1};
+}
+RowShape split_shape(int64_t rows, int64_t nvec, bool bf16) {
+    if (nvec <= kWave) return {1, 1};
+    if (bf16 && rows * nvec * 16 > kMallBytes / 8) return {2, 1};
+    if (nvec <= 2 * kWave) return rows <= 512 ? RowShape{1, 1} : RowShape{1, 2};
+    if (nvec <= 4 * kWave || rows <= 512 || (rows <= 1024 && nvec > 8 * kWave)) return {1, 4};
+    if (nvec <= 8 * kWave) return {2, 4};
+    return {2, 1};
+}
 bool elem_at(const void* p, int64_t esz) { return reinterpret_cast<uintptr_t>(p) % esz == 0; }
+
+// The vectors that a row is moved in; 0 for rows that go element by element
+// in a block of 4 waves: those off their elements' addresses, those whose
+// pieces no dispatch counts, and few short ones that end in a tail of
+// elements, where a vector and then the tail is the longer wait (64 x 257 bf16
+// split 3.5 us against 3.0; four microbatches of 256 x 257 24.1 against 21.6).
+int64_t row_vecs(int64_t rows, int64_t d, int64_t esz, bool at_elems) {
+    const int64_t nvec = d * esz / 16;
+    const bool few_tails = rows <= (esz == 2 ? 1024 : 256) && d <= 512 && d * esz % 16 != 0;
+    return at_elems && !few_tails && nvec < 0xFFFF0000LL ? nvec : 0;
+}
 
 }  // namespace
 }  // namespace ely
@@ -209,13 +252,24 @@ extern "C" int ely_rows_fold(void* acc, const void* a, const int64_t* a_rows, co
         if (b_rows && !b) fail(ELY_EINVAL, "ely_rows_fold: b_rows without b");
         if (b && !b_rows && b_total < n_idx) fail(ELY_EINVAL, "ely_rows_fold: a compact b holds one row per index");
         const int64_t esz = dtype == ELY_BF16 ? 2 : 4;
-        const int vec = elem_at(acc, esz) && elem_at(a, esz) && elem_at(b, esz) ? 1 : 0;
-        const dim3 grid = rows_grid(n_idx, d, esz, vec, kFoldVecs, "ely_rows_fold");
-        const bool stream_it = 3 * n_idx * d * esz > kMallBytes;
-        const auto kern = dtype == ELY_BF16 ? (stream_it ? rows_fold_kernel<true, true> : rows_fold_kernel<true, false>)
-                                            : (stream_it ? rows_fold_kernel<false, true> : rows_fold_kernel<false, false>);
-        hipLaunchKernelGGL(kern, grid, dim3(kWave), 0, static_cast<hipStream_t>(stream), acc, a, a_rows, b, b_rows, idx,
-                           n_idx, n_rows, a_total, b ? b_total : 0, d, first ? 1 : 0, vec);
+        const int64_t nvec = row_vecs(n_idx, d, esz, elem_at(acc, esz) && elem_at(a, esz) && elem_at(b, esz));
+        const int vec = nvec > 0;
+        const auto launch = [&](auto kern, int v, int w) {
+            const dim3 grid = rows_grid(n_idx, nvec, kWave * v * w, kWave * w);
+            hipLaunchKernelGGL(kern, grid, dim3(kWave * w), 0, static_cast<hipStream_t>(stream), acc, a, a_rows, b, b_rows,
+                               idx, n_idx, n_rows, a_total, b ? b_total : 0, d, first ? 1 : 0, vec);
+        };
+        const auto shape = [&](auto bf16) {
+            constexpr bool B = decltype(bf16)::value;
+            if (3 * n_idx * d * esz > kMallBytes) return launch(rows_fold_kernel<B, 1, 1, true>, 1, 1);
+            const RowShape sh = vec ? fold_shape(n_idx, nvec, B) : RowShape{1, 4};
+            if (sh.v == 2 && sh.w == 4) launch(rows_fold_kernel<B, 2, 4, false>, 2, 4);
+            else if (sh.v == 2) launch(rows_fold_kernel<B, 2, 2, false>, 2, 2);
+            else if (sh.w == 4) launch(rows_fold_kernel<B, 1, 4, false>, 1, 4);
+            else if (sh.w == 2) launch(rows_fold_kernel<B, 1, 2, false>, 1, 2);
+            else launch(rows_fold_kernel<B, 1, 1, false>, 1, 1);
+        };
+        dtype == ELY_BF16 ? shape(std::true_type()) : shape(std::false_type());
         check_launch("rows_fold_kernel");
     });
 }
@@ -229,13 +283,24 @@ extern "C" int ely_rows_split(void* acc, const void* a, const int32_t* slot, voi
         if (n_rows == 0 || d == 0) return;
         if (!acc || !a || !slot || (n_held && !held_out)) fail(ELY_EINVAL, "ely_rows_split: null pointer");
         const int64_t esz = dtype == ELY_BF16 ? 2 : 4;
-        const int vec = elem_at(acc, esz) && elem_at(a, esz) && elem_at(held_out, esz) ? 1 : 0;
-        const dim3 grid = rows_grid(n_rows, d, esz, vec, kSplitVecs, "ely_rows_split");
-        const bool stream_it = 2 * n_rows * d * esz > kMallBytes;
-        const auto kern = dtype == ELY_BF16 ? (stream_it ? rows_split_kernel<true, true> : rows_split_kernel<true, false>)
-                                            : (stream_it ? rows_split_kernel<false, true> : rows_split_kernel<false, false>);
-        hipLaunchKernelGGL(kern, grid, dim3(kWave), 0, static_cast<hipStream_t>(stream), acc, a, slot, held_out, n_rows,
-                           n_held, d, first ? 1 : 0, vec);
+        const int64_t nvec = row_vecs(n_rows, d, esz, elem_at(acc, esz) && elem_at(a, esz) && elem_at(held_out, esz));
+        const int vec = nvec > 0;
+        const auto launch = [&](auto kern, int v, int w) {
+            const dim3 grid = rows_grid(n_rows, nvec, kWave * v * w, kWave * w);
+            hipLaunchKernelGGL(kern, grid, dim3(kWave * w), 0, static_cast<hipStream_t>(stream), acc, a, slot, held_out,
+                               n_rows, n_held, d, first ? 1 : 0, vec);
+        };
+        const auto shape = [&](auto bf16) {
+            constexpr bool B = decltype(bf16)::value;
+            if (2 * n_rows * d * esz > kMallBytes) return launch(rows_split_kernel<B, 2, 1, true>, 2, 1);
+            const RowShape sh = vec ? split_shape(n_rows, nvec, B) : RowShape{1, 4};
+            if (sh.v == 2 && sh.w == 4) launch(rows_split_kernel<B, 2, 4, false>, 2, 4);
+            else if (sh.v == 2) launch(rows_split_kernel<B, 2, 1, false>, 2, 1);
+            else if (sh.w == 4) launch(rows_split_kernel<B, 1, 4, false>, 1, 4);
+            else if (sh.w == 2) launch(rows_split_kernel<B, 1, 2, false>, 1, 2);
+            else launch(rows_split_kernel<B, 1, 1, false>, 1, 1);
+        };
+        dtype == ELY_BF16 ? shape(std::true_type()) : shape(std::false_type());
         check_launch("rows_split_kernel");
     });
 }
