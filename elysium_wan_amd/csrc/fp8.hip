@@ -611,9 +611,15 @@ __global__ __launch_bounds__(kQBlock) void quant_split_kernel(const void* __rest
     uint4 buf[Seg<BF16>::VPL];
     if (vec) load_segment<BF16>(static_cast<const char*>(x) + row * cols * SegAt<BF16>::ESZ, at, lane, buf);
     uint32_t m = 0;
+    if (bpr == 1) {
+        // short rows: the one word, without the butterfly (8.4 M rows of 4 bf16
+        // 4171 -> 3828 us; longer rows the same)
+        m = partial[row];
+    } else {
 #pragma unroll 4
-    for (int64_t i = lane; i < bpr; i += kWave) m = max(m, partial[row * bpr + i]);
-    m = wave_max_u32(m);
+        for (int64_t i = lane; i < bpr; i += kWave) m = max(m, partial[row * bpr + i]);
+        m = wave_max_u32(m);
+    }
     const RowScale rs = row_scale<FMT>(to_f32_bits<BF16>(m), BF16, BF16);
     if (seg == 0 && lane == 0 && k) k[row] = rs.k;
     if (vec && rs.fast) {
