@@ -56,9 +56,20 @@ def test_ragged_dequantize_with_a_distinct_exponent_per_row(oracle, fmt, cols):
     """Every code, neighbouring rows' exponents different and some outside
     the instruction path, so that a vector holding the end of one row and the
     start of the next shows a wrong one; q off its boundary too."""
+    _ragged_dequantize_equals_the_oracle(oracle, fmt, cols, max(3, (5 * 1024 + 7) // cols))
+
+
+# both sides of the number of rows up to which narrow fp32 results go row by row
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("cols", [8, 9, 13, 31, 100, 255, 256, 257])
+@pytest.mark.parametrize("rows", [1, 3, 33, 2048, 2049])
+def test_ragged_dequantize_of_few_and_of_many_rows(oracle, fmt, cols, rows):
+    _ragged_dequantize_equals_the_oracle(oracle, fmt, cols, rows)
+
+
+def _ragged_dequantize_equals_the_oracle(oracle, fmt, cols, rows):
     from elysium_wan_amd import fp8
 
-    rows = max(3, (5 * 1024 + 7) // cols)
     rng = np.random.default_rng(cols)
     codes = ((np.arange(rows * cols, dtype=np.int64) * 37 + 11) % 256).astype(np.uint8)
     kk = rng.integers(-140, 141, rows).astype(np.int32)
