@@ -452,7 +452,10 @@ PyObject* py_clip(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const int64_t wn = ws.numel();
     void* s = stream_of(dev);
     if (unlocked([&] { return ely_grad_norm_clip(G.data(), ns, (float)max_norm, rp, wp, wn, s); }) != ELY_OK) Py_RETURN_NONE;
-    return THPVariable_Wrap(res.select(0, 2));
+    // a tensor of its own over the result's memory: as a view of it, detach_() would be refused
+    Tensor total = at::empty({0}, res.options());
+    total.set_(res.storage(), 2, {}, {});
+    return THPVariable_Wrap(std::move(total));
     END_HANDLE_TH_ERRORS
 }
 

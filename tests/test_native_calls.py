@@ -194,3 +194,17 @@ def test_a_failed_check_leaves_state_and_tensors_alone():
             opt.step(grads=good[:2] + [bad])
         assert [float(opt.state[i]["step"]) for i in range(3)] == [1.0] * 3
         assert all(torch.equal(p.detach(), b) for p, b in zip(ps, before))
+
+
+@pytest.mark.gpu
+def test_the_clips_total_is_a_tensor_of_its_own():
+    """As the Python path's clone: no view, which could not be detached in place."""
+    from elysium_wan_amd import optim
+
+    p = torch.zeros(300, device="cuda")
+    p.grad = torch.full((300,), 2.0, device="cuda")
+    total = optim.clip_grad_norm_([p], 1.0)
+    assert not total._is_view() and total.dim() == 0 and total.dtype == torch.float32
+    total.detach_()
+    again = optim.clip_grad_norm_([p], 1.0)
+    assert abs(float(total) - 2.0 * 300**0.5) < 1e-4 and abs(float(again) - 1.0) < 1e-5
