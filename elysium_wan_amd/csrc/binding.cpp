@@ -264,9 +264,12 @@ PyObject* py_fold_add(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// A tensor that the call only reads, and one that it writes: of a lazy copy
+// the latter is given memory of its own first, as Tensor.data_ptr() does.
 ely_tensor entry(const Tensor& t) {
     return ely_tensor{const_cast<void*>(t.const_data_ptr()), t.numel(), dtype_code(t), 0};
 }
+ely_tensor written(const Tensor& t) { return ely_tensor{t.mutable_data_ptr(), t.numel(), dtype_code(t), 0}; }
 
 // Fails of adamw_step and clip that the library reported: (status, which call).
 PyObject* status(int rc, int which) { return Py_BuildValue("(ii)", rc, which); }
@@ -331,12 +334,12 @@ PyObject* py_adamw_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         } else {
             const Tensor* c = kernel_tensor(co);
             if (!c) Py_RETURN_NONE;
-            C.push_back(entry(*c));
+            C.push_back(written(*c));
         }
-        P.push_back(entry(*p));
+        P.push_back(written(*p));
         G.push_back(entry(*g));
-        M.push_back(entry(*m));
-        V.push_back(entry(*v));
+        M.push_back(written(*m));
+        V.push_back(written(*v));
         idx.push_back(i);
         n_bf16 += g->scalar_type() == at::kBFloat16;
     }
@@ -440,7 +443,7 @@ PyObject* py_clip(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (!plain_tensor(g) || !g.is_cuda() || !g.is_contiguous() || dtype_code(g) < 0) Py_RETURN_NONE;
         if (dev < 0) dev = (c10::DeviceIndex)g.get_device();
         if (g.get_device() != dev) Py_RETURN_NONE;
-        G.push_back(entry(g));
+        G.push_back(written(g));
     }
     if (G.empty() || G.size() > INT32_MAX || c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().device_index() != dev) Py_RETURN_NONE;
     const int32_t ns = (int32_t)G.size();

@@ -208,3 +208,33 @@ def test_the_clips_total_is_a_tensor_of_its_own():
     total.detach_()
     again = optim.clip_grad_norm_([p], 1.0)
     assert abs(float(total) - 2.0 * 300**0.5) < 1e-4 and abs(float(again) - 1.0) < 1e-5
+
+
+@pytest.mark.gpu
+def test_what_a_call_writes_is_not_shared_with_a_lazy_copy():
+    """torch's lazy copies share memory until one of them is written."""
+    from elysium_wan_amd import optim
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    grad = torch.randn(300, generator=g, device="cuda")
+    p = torch.zeros(300, device="cuda")
+    first, p.grad = grad.clone(), torch._lazy_clone(grad)
+    optim.clip_grad_norm_([p], 0.5)
+    assert torch.equal(grad, first) and not torch.equal(p.grad, first)
+
+    got = []
+    for lazy in (False, True):
+        q = torch.ones(300, device="cuda", requires_grad=True)
+        opt = optim.FusedAdamW([q], lr=1e-3, working_copy=True)
+        opt.step(grads=[grad])
+        tensors = [q.detach(), opt.state[0]["exp_avg"], opt.state[0]["exp_avg_sq"], opt.working_copies[0]]
+        if lazy:
+            kept = [t.clone() for t in tensors]
+            shared = [torch._lazy_clone(t) for t in tensors]
+            q.data = torch._lazy_clone(shared[0])
+            opt._st[0]["exp_avg"], opt._st[0]["exp_avg_sq"] = torch._lazy_clone(shared[1]), torch._lazy_clone(shared[2])
+            opt.working_copies[0] = torch._lazy_clone(shared[3])
+        opt.step(grads=[grad])
+        got.append([q.detach(), opt.state[0]["exp_avg"], opt.state[0]["exp_avg_sq"], opt.working_copies[0]])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert all(torch.equal(a, b) for a, b in zip(kept, shared))
