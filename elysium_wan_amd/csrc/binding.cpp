@@ -271,6 +271,28 @@ ely_tensor entry(const Tensor& t) {
 }
 ely_tensor written(const Tensor& t) { return ely_tensor{t.mutable_data_ptr(), t.numel(), dtype_code(t), 0}; }
 
+// References to the objects whose memory a call's tables name, held until its
+// launches are queued: the caller's lists and the state may change meanwhile, in
+// consts() or in another thread while the interpreter lock is released.
+class Held {
+public:
+    Held() = default;
+    Held(const Held&) = delete;
+    Held& operator=(const Held&) = delete;
+    ~Held() {
+        for (PyObject* o : objects_) Py_DECREF(o);
+    }
+    void reserve(size_t n) { objects_.reserve(n); }
+    PyObject* add(PyObject* o) {
+        objects_.push_back(o);
+        Py_INCREF(o);
+        return o;
+    }
+
+private:
+    std::vector<PyObject*> objects_;
+};
+
 // Fails of adamw_step and clip that the library reported: (status, which call).
 PyObject* status(int rc, int which) { return Py_BuildValue("(ii)", rc, which); }
 
@@ -302,6 +324,8 @@ PyObject* py_adamw_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 
     static PyObject* k_m = PyUnicode_InternFromString("exp_avg");
     static PyObject* k_v = PyUnicode_InternFromString("exp_avg_sq");
+    Held held;
+    held.reserve((size_t)n * 6);
     std::vector<ely_tensor> P, G, A, M, V, C;
     std::vector<Py_ssize_t> idx;
     for (auto* v : {&P, &G, &M, &V, &C}) v->reserve(n);
@@ -311,11 +335,11 @@ PyObject* py_adamw_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject* go = PyList_GET_ITEM(grads, i);
         if (go == Py_None) continue;
-        const Tensor *p = kernel_tensor(PyList_GET_ITEM(params, i)), *g = kernel_tensor(go);
+        const Tensor *p = kernel_tensor(held.add(PyList_GET_ITEM(params, i))), *g = kernel_tensor(held.add(go));
         if (!p || !g || p->scalar_type() != at::kFloat || p->get_device() != dev || g->get_device() != dev || g->sizes() != p->sizes())
             Py_RETURN_NONE;
         if (fold) {
-            const Tensor* ac = kernel_tensor(PyList_GET_ITEM(accs, i));
+            const Tensor* ac = kernel_tensor(held.add(PyList_GET_ITEM(accs, i)));
             if (!ac || ac->scalar_type() != at::kFloat || ac->get_device() != dev || ac->sizes() != p->sizes()) Py_RETURN_NONE;
             A.push_back(entry(*ac));
         }
@@ -326,13 +350,13 @@ PyObject* py_adamw_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (!st && PyErr_Occurred()) return nullptr;
         if (!st || !PyDict_CheckExact(st)) Py_RETURN_NONE;
         PyObject *mo = PyDict_GetItem(st, k_m), *vo = PyDict_GetItem(st, k_v);
-        const Tensor *m = mo ? kernel_tensor(mo) : nullptr, *v = vo ? kernel_tensor(vo) : nullptr;
+        const Tensor *m = mo ? kernel_tensor(held.add(mo)) : nullptr, *v = vo ? kernel_tensor(held.add(vo)) : nullptr;
         if (!m || !v || m->scalar_type() != at::kFloat || v->scalar_type() != at::kFloat) Py_RETURN_NONE;
         PyObject* co = copy ? PyList_GET_ITEM(copies, i) : Py_None;
         if (co == Py_None) {
             C.push_back(ely_tensor{nullptr, 0, ELY_BF16, 0});
         } else {
-            const Tensor* c = kernel_tensor(co);
+            const Tensor* c = kernel_tensor(held.add(co));
             if (!c) Py_RETURN_NONE;
             C.push_back(written(*c));
         }
@@ -432,7 +456,10 @@ PyObject* py_clip(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     }
     const Py_ssize_t n = PySequence_Fast_GET_SIZE(a[0]);
+    // the gradients themselves: .grad may be cleared while the interpreter lock is released
+    std::vector<Tensor> held;
     std::vector<ely_tensor> G;
+    held.reserve(n);
     G.reserve(n);
     c10::DeviceIndex dev = -1;
     for (Py_ssize_t i = 0; i < n; ++i) {
@@ -444,6 +471,7 @@ PyObject* py_clip(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (dev < 0) dev = (c10::DeviceIndex)g.get_device();
         if (g.get_device() != dev) Py_RETURN_NONE;
         G.push_back(written(g));
+        held.push_back(g);
     }
     if (G.empty() || G.size() > INT32_MAX || c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().device_index() != dev) Py_RETURN_NONE;
     const int32_t ns = (int32_t)G.size();

@@ -8,6 +8,8 @@ import os
 import shutil
 import subprocess
 import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -238,3 +240,80 @@ def test_what_a_call_writes_is_not_shared_with_a_lazy_copy():
         got.append([q.detach(), opt.state[0]["exp_avg"], opt.state[0]["exp_avg_sq"], opt.working_copies[0]])
     assert all(torch.equal(a, b) for a, b in zip(*got))
     assert all(torch.equal(a, b) for a, b in zip(kept, shared))
+
+
+@pytest.mark.gpu
+def test_the_step_keeps_its_tensors_until_it_is_queued():
+    """The caller's lists emptied in the middle of the call, and their memory
+    asked for again at once."""
+    from elysium_wan_amd import optim
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    grads, accs = ([torch.randn(70001, generator=g, device="cuda") for _ in range(3)] for _ in range(2))
+    got = []
+    for emptied in (False, True):
+        ps = [torch.ones(70001, device="cuda", requires_grad=True) for _ in grads]
+        opt = optim.FusedAdamW(ps, lr=1e-3, max_norm=1.0)
+        opt.step(grads=grads)
+        gl, al, junk, consts = [t.clone() for t in grads], [t.clone() for t in accs], [], opt._consts
+
+        def in_the_middle(*args):
+            gl[:], al[:] = [None] * 3, [None] * 3
+            junk.extend(torch.full((70001,), 1e6, device="cuda") for _ in range(12))
+            return consts(*args)
+
+        if emptied:
+            opt._consts = in_the_middle
+        opt.step(grads=gl, acc=al)
+        assert len(junk) == 12 * emptied
+        got.append([t for i, p in enumerate(ps) for t in (p.detach(), opt.state[i]["exp_avg"], opt.state[i]["exp_avg_sq"])] + [opt.grad_norm()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.gpu
+def test_the_clip_keeps_its_gradients_until_it_is_queued():
+    """The clip of a long list waits for a slot of the upload ring, the
+    interpreter lock released, while another thread clears the gradients and
+    asks for their memory again."""
+    from elysium_wan_amd import optim
+
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    torch.cuda._sleep(1000)
+    start.record()
+    torch.cuda._sleep(1_000_000)
+    end.record()
+    end.synchronize()
+    busy = int(1_000_000 * 400 / max(start.elapsed_time(end), 1e-2))  # 0.4 s
+
+    def params(value):
+        ps = [torch.zeros(5000, device="cuda") for _ in range(60)]
+        for p in ps:
+            p.grad = torch.full((5000,), value, device="cuda")
+        return ps
+
+    ps, others = params(3.0), params(1.0)
+    optim.clip_grad_norm_(others, 1e9)
+    torch.cuda.synchronize()
+    go, junk, cleared = threading.Event(), [], []
+
+    def clear():
+        go.wait(30)
+        time.sleep(0.05)
+        for p in ps:
+            p.grad = None
+        junk.extend(torch.full((5000,), 7.0, device="cuda") for _ in range(120))
+        cleared.append(time.monotonic())
+
+    t = threading.Thread(target=clear)
+    t.start()
+    torch.cuda._sleep(busy)
+    for _ in range(8):  # every slot of the ring behind the busy stream
+        optim.clip_grad_norm_(others, 1e9)
+    go.set()
+    total = optim.clip_grad_norm_(ps, 1.0)
+    done = time.monotonic()
+    t.join()
+    torch.cuda.synchronize()
+    assert cleared[0] < done, "the gradients were to be cleared during the call"
+    assert abs(float(total) - 3.0 * (60 * 5000) ** 0.5) < 1e-2
+    assert all(bool((j == 7.0).all()) for j in junk)
