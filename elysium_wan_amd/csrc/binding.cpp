@@ -75,7 +75,10 @@ void* stream_of(c10::DeviceIndex dev) { return c10::hip::getCurrentHIPStreamMasq
 // Scratch buffers, one per device and stream: calls on one stream are
 // ordered, so reuse is safe; when one grows, the old buffer returns to
 // torch's allocator, which reuses it only after work already queued on that
-// stream.  Never destroyed: the GPU runtime ends before static objects do.
+// stream.  The map is never destroyed: the GPU runtime ends before static
+// objects do.  Nothing is allocated or freed under the mutex: the allocator
+// may run Python (a memory trace) and so let another thread go on to wait
+// for the mutex with the interpreter lock held.
 std::mutex g_ws_mu;
 std::map<std::pair<int, void*>, Tensor>& workspaces() {
     static auto* m = new std::map<std::pair<int, void*>, Tensor>();
@@ -85,11 +88,20 @@ std::map<std::pair<int, void*>, Tensor>& workspaces() {
 Tensor workspace(c10::DeviceIndex dev, int64_t nbytes) {
     nbytes = std::max<int64_t>(nbytes, 256);
     const std::pair<int, void*> key(dev, stream_of(dev));
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mu);
+        const auto it = workspaces().find(key);
+        if (it != workspaces().end() && it->second.numel() >= nbytes) return it->second;
+    }
+    const Tensor buf = at::empty({std::max<int64_t>(nbytes, 1 << 20)},
+                                 at::TensorOptions().dtype(at::kByte).device(c10::Device(at::kCUDA, dev)));
+    Tensor old;  // outlives the lock
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    Tensor& buf = workspaces()[key];
-    if (!buf.defined() || buf.numel() < nbytes)
-        buf = at::empty({std::max<int64_t>(nbytes, 1 << 20)},
-                        at::TensorOptions().dtype(at::kByte).device(c10::Device(at::kCUDA, dev)));
+    Tensor& kept = workspaces()[key];
+    if (!kept.defined() || kept.numel() < buf.numel()) {
+        old = std::move(kept);
+        kept = buf;
+    }
     return buf;
 }
 

@@ -317,3 +317,38 @@ def test_the_clip_keeps_its_gradients_until_it_is_queued():
     assert cleared[0] < done, "the gradients were to be cleared during the call"
     assert abs(float(total) - 3.0 * (60 * 5000) ** 0.5) < 1e-2
     assert all(bool((j == 7.0).all()) for j in junk)
+
+
+@pytest.mark.gpu
+def test_a_workspace_grows_while_another_thread_asks_for_one():
+    """The allocator may run Python, here a memory trace that waits for a
+    second thread's call: that call must not wait for the first one's.  In a
+    process of its own, for the trace stays on."""
+    r = subprocess.run([sys.executable, "-u", "-c", """
+import threading, torch
+from torch.cuda import _gpu_trace
+from elysium_wan_amd import _lib
+
+N = _lib.load_native()
+N.workspace(0, 1)
+inside, done, waited = threading.Event(), threading.Event(), []
+
+def traced(ptr):
+    if not inside.is_set():
+        inside.set()
+        waited.append(done.wait(20))
+
+def second():
+    inside.wait(20)
+    N.workspace(0, 1)
+    done.set()
+
+_gpu_trace.register_callback_for_memory_allocation(traced)
+torch._C._activate_gpu_trace()
+t = threading.Thread(target=second)
+t.start()
+grown = N.workspace(0, 8 << 20)
+t.join()
+assert waited == [True] and grown.numel() >= 8 << 20 and N.workspace(0, 1).data_ptr() == grown.data_ptr()
+"""], cwd=ROOT, capture_output=True, text=True, timeout=90)
+    assert r.returncode == 0, r.stdout + r.stderr
