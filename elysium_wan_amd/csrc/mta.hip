@@ -973,16 +973,17 @@ static void clip_scale(const NormLaunch& nl, const float* coef_dev, void* stream
     if (nl.tiles == 0) return;
     // one wave per tile, in whole blocks; the blocks capped so that the
     // dispatch's work-items stay within 2^32 - 1 (the waves stride past that)
-    const int64_t waves = std::min<int64_t>(nl.tiles, mt_blocks(ELY_CLIP_BPC) * (kBlock / kWave));
-    const int64_t groups = std::min<int64_t>((waves + kBlock / kWave * kXcds - 1) / (kBlock / kWave * kXcds),
-                                             0xFFFFFFFFLL / (kBlock * kXcds));
-    const int64_t blocks = groups * kXcds;
+    const int64_t most = std::min<int64_t>(mt_blocks(ELY_CLIP_BPC), 0xFFFFFFFFLL / kBlock);
+    int64_t blocks = std::min<int64_t>((nl.tiles + kBlock / kWave - 1) / (kBlock / kWave), most);
     // The norm read its tiles first to last; a list the 256 MB MALL holds is
     // scaled last to first, so that it begins on what the L2s hold too, with a
     // block's tiles on the XCD that summed them (the scale of 88 MB of fp32
     // 31.8 -> 26.4 us, of 134 MB of bf16 39.9 -> 37.7).  Larger lists measured
-    // the same or worse that way (516 MB of fp32 155 -> 157 us).
-    const int32_t last_first = nl.tiles * nl.tile * (nl.dt == ELY_BF16 ? 2 : 4) <= (int64_t)256 << 20;
+    // the same or worse that way (516 MB of fp32 155 -> 157 us).  It takes
+    // blocks in whole groups of kXcds, which a cap may not leave room for.
+    const int64_t grouped = (blocks + kXcds - 1) / kXcds * kXcds;
+    const int32_t last_first = grouped <= most && nl.tiles * nl.tile * (nl.dt == ELY_BF16 ? 2 : 4) <= (int64_t)256 << 20;
+    if (last_first) blocks = grouped;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (nl.dtable) {
         const ClipKernel k = nl.tile == kNormTile ? pick_clip<kNormTile>(nl.dt) : pick_clip<kNormSmallTile>(nl.dt);

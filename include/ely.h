@@ -293,7 +293,7 @@ int ely_scale_inplace(const ely_tensor* tensors, int32_t n, const float* coef_de
  * over PCIe.  ELY_EINVAL if `host` is not such memory. */
 int ely_host_device_pointer(const void* host, void** device);
 
-/* Cap on the blocks one multi-tensor launch (grad-norm, AdamW) may use; 0
+/* Cap on the blocks one multi-tensor launch (grad-norm, clip, AdamW) may use; 0
  * restores each kernel's own grid.  For tuning and for the tests
  * that prove results do not depend on the grid.  Process-wide. */
 int ely_set_max_blocks(int32_t max_blocks);

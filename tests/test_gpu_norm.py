@@ -199,3 +199,36 @@ def test_norm_over_both_load_kinds_is_bitwise_stable_across_grids():
             _lib.load().ely_set_max_blocks(0)
         assert abs(r[0] - exact) <= 1e-8 * exact
     assert all(np.array_equal(runs[0], r) for r in runs[1:])
+
+
+@pytest.mark.parametrize("cap", [1, 5, 8, 13])
+def test_the_clip_keeps_to_the_cap_on_blocks(cap, tmp_path):
+    """ely_set_max_blocks bounds the scale's grid too (read from a profile),
+    and the scaled gradients do not depend on it."""
+    import json
+
+    from elysium_wan_amd import _lib, optim
+    from torch.profiler import ProfilerActivity, profile
+
+    gen = torch.Generator(device="cuda").manual_seed(cap)
+    values = [torch.randn(n, device="cuda", generator=gen) for n in (1 << 20, 70001, 3)]
+    got = []
+    for c in (0, cap):
+        ps = [torch.zeros_like(v) for v in values]
+        for p, v in zip(ps, values):
+            p.grad = v.clone()
+        say("clip under a cap of", c)
+        _lib.check(_lib.load().ely_set_max_blocks(c), "cap")
+        try:
+            with profile(activities=[ProfilerActivity.CUDA]) as prof:
+                got.append([optim.clip_grad_norm_(ps, 1.0)] + [p.grad for p in ps])
+                torch.cuda.synchronize()
+        finally:
+            _lib.load().ely_set_max_blocks(0)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    prof.export_chrome_trace(str(tmp_path / "trace.json"))
+    grids = [e["args"]["grid"][0] for e in json.loads((tmp_path / "trace.json").read_text())["traceEvents"]
+             if e.get("cat") == "kernel" and "clip_scale" in e["name"]]
+    if not grids:
+        pytest.skip("the profiler reports no launches here")
+    assert max(grids) <= cap
