@@ -98,29 +98,37 @@ def test_per_tensor_of_any_length_equals_the_oracle(oracle, dname, n):
         _codec_equals_the_oracle(oracle, x.reshape(1, n), "e4m3" if off else "e5m2")
 
 
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("dname", ["bf16", "f32"])
 @pytest.mark.parametrize("off", [0, 3])
-def test_a_ragged_tensor_past_the_guess_size_equals_torch(off):
-    """An odd length of over 64 MiB, its largest value in the vector that
-    overlaps the last whole segment, against torch's own ops on this GPU."""
+def test_a_ragged_tensor_past_the_guess_size_equals_torch(dname, fmt, off):
+    """An odd length of over 64 MiB, its largest value (infinities and NaN
+    too) in the vector that overlaps the last whole segment, which the guess
+    does not sample, against torch's own ops on this GPU."""
     from elysium_wan_amd import fp8
 
-    n = (1 << 25) + 2048 + 5
+    dt, (f8, e) = DT[dname], fp8.FORMATS[fmt]
+    n = (1 << (25 if dname == "bf16" else 24)) + 2048 + 5
+    assert (n // 2048 - 1) % 61 != 0 and (n // 2048) % 61 != 0
     g = torch.Generator(device="cuda").manual_seed(off)
-    x = torch.randn(n + off, generator=g, device="cuda").bfloat16()[off:]
-    for top in (None, 1e4, "rising"):
+    x = torch.randn(n + off, generator=g, device="cuda").to(dt)[off:]
+    for top in (None, 1e4, float("inf"), float("-inf"), float("nan"), "rising"):
         if top == "rising":  # every segment that the guess does not sample exceeds those it does
             x[: n // 2048 * 2048].view(-1, 2048)[::61] *= 2.0**-5
             x[n - 2] = 0.25
         elif top is not None:
             x[n - 2] = top
-        say("fp8 ragged guess", off, top)
-        q, k = fp8.quantize(x, "e4m3", per_tensor=True)
-        amax = x.abs().max().float()
-        kref = int(torch.frexp(amax).exponent) - 8
+        say("fp8 ragged guess", dname, fmt, off, top)
+        q, k = fp8.quantize(x, fmt, per_tensor=True)
+        back = fp8.roundtrip(x, fmt, per_tensor=True)
+        amax = x.abs().max().float().cpu()
+        # frexp's exponent of an infinity is 0; a NaN maximum scales by 1 (model/fp8.py:36-38)
+        kref = 0 if amax.isnan() else -e if amax.isinf() else int(torch.frexp(amax).exponent) - e
         assert int(k) == kref
-        qref = (x * 2.0**-kref).to(torch.float8_e4m3fn)
+        qref = (x * torch.tensor(2.0**-kref, dtype=dt, device="cuda")).to(f8)
         assert torch.equal(q.view(torch.uint8), qref.view(torch.uint8))
-        assert torch.equal(fp8.roundtrip(x, "e4m3", per_tensor=True), qref.to(torch.bfloat16) * 2.0**kref)
+        want = qref.to(dt) * torch.tensor(2.0**kref, dtype=dt, device="cuda")
+        assert torch.equal(torch.nan_to_num(back, nan=7.0), torch.nan_to_num(want, nan=7.0)) and torch.equal(back.isnan(), want.isnan())
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 257, 4099])

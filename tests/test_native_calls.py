@@ -151,8 +151,8 @@ def test_plain_calls_are_taken_and_equal_the_python_path(monkeypatch):
 
     monkeypatch.setattr(_lib, "_native", Spy())
     fast = calls()
-    # all but the optimizer's first step, which makes its state, go the native way
-    assert [t for t in taken if not t[1]] == [("adamw_step", False)] or not [t for t in taken if not t[1]]
+    # the optimizer's first step, which makes its state, does not ask; every call that does is taken
+    assert all(ok for _, ok in taken) and [n for n, _ in taken].count("adamw_step") == 5
     assert {n for n, ok in taken if ok} == {"quantize", "roundtrip", "dequantize", "cast_bf16", "widen_bf16", "fold_add", "adamw_step", "clip"}
     monkeypatch.setattr(_lib, "_native", Off())
     slow = calls()
