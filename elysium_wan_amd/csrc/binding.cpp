@@ -502,8 +502,12 @@ PyObject* py_clip(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// abi_version(): of the library that these calls run in.
+PyObject* py_abi_version(PyObject*, PyObject*) { return PyLong_FromLong(ely_abi_version()); }
+
 #define FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)), METH_FASTCALL
 PyMethodDef kMethods[] = {
+    {"abi_version", py_abi_version, METH_NOARGS, "abi_version()"},
     {"workspace", FAST(py_workspace), "workspace(device index, nbytes)"},
     {"quantize", FAST(py_quantize), "quantize(x, fmt, per_tensor)"},
     {"roundtrip", FAST(py_roundtrip), "roundtrip(x, fmt, per_tensor)"},

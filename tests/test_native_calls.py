@@ -84,20 +84,48 @@ assert _lib.load_native().quantize(torch.zeros(2, 8), "e4m3", False) is None and
 """)
 
 
-def test_a_library_rebuilt_after_the_import_is_the_one_that_runs(tmp_path):
-    _copy_of_the_package(tmp_path, *LIBRARIES)
-    _run(tmp_path, """
+# as a rebuild leaves the files: new ones at the old paths
+REPLACE = """
 import os, shutil
+def replaced(name, new):
+    shutil.copy(new, "new")
+    os.replace("new", "elysium_wan_amd/" + name)
+def mapped(name):
+    return {line.split()[4] for line in open("/proc/self/maps") if "/elysium_wan_amd/" in line and line.rstrip().endswith(name)}
+"""
+
+
+@pytest.mark.parametrize("first", ["load", "load_native"])
+def test_a_library_rebuilt_after_the_import_is_the_one_that_runs(tmp_path, first):
+    """The new library answers through ctypes and through the new _native, and
+    a later rebuild changes nothing for this process."""
+    _copy_of_the_package(tmp_path, *LIBRARIES)
+    stub = tmp_path / "stub.c"
+    stub.write_text("\n".join(f"int {n}(void) {{ return {77 if n == 'ely_abi_version' else 0}; }}" for n in _lib.EXPORTS))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "stub.so"), str(stub)], check=True)
+    _run(tmp_path, REPLACE + f"""
 import elysium_wan_amd
 from elysium_wan_amd import _lib, accumulate, boundary, f32_planes, fp8, fp8_planes, optim, pieces, planes
+replaced("libelyhip.so", "stub.so")
+replaced("_native.so", {os.path.join(PACKAGE, "_native.so")!r})
+_lib.{first}()
+N = _lib.load_native()
+assert _lib.load().ely_abi_version() == 77 and N.abi_version() == 77
+for name in ("libelyhip.so", "_native.so"):
+    assert str(os.stat("elysium_wan_amd/" + name).st_ino) in mapped(name), name
+replaced("libelyhip.so", {os.path.join(PACKAGE, "libelyhip.so")!r})
+assert _lib.load().ely_abi_version() == 77 and _lib.load_native() is N
+""")
 
+
+def test_an_unchanged_library_is_mapped_once(tmp_path):
+    _copy_of_the_package(tmp_path, *LIBRARIES)
+    _run(tmp_path, REPLACE + """
+from elysium_wan_amd import _lib
+N = _lib.load_native()
+assert N.abi_version() == _lib.load().ely_abi_version() == 1
 for name in ("libelyhip.so", "_native.so"):
-    shutil.copy("elysium_wan_amd/" + name, "new")
-    os.replace("new", "elysium_wan_amd/" + name)
-_lib.load(), _lib.load_native()
-for name in ("libelyhip.so", "_native.so"):
-    mapped = {line.split()[4] for line in open("/proc/self/maps") if "/elysium_wan_amd/" + name in line}
-    assert mapped == {str(os.stat("elysium_wan_amd/" + name).st_ino)}, (name, mapped)
+    assert mapped(name) == {str(os.stat("elysium_wan_amd/" + name).st_ino)}, name
 """)
 
 
@@ -352,3 +380,23 @@ t.join()
 assert waited == [True] and grown.numel() >= 8 << 20 and N.workspace(0, 1).data_ptr() == grown.data_ptr()
 """], cwd=ROOT, capture_output=True, text=True, timeout=90)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_kernels_of_a_library_rebuilt_after_the_import_run(tmp_path):
+    _copy_of_the_package(tmp_path, *LIBRARIES)
+    _run(tmp_path, REPLACE + f"""
+import torch
+from elysium_wan_amd import _lib, fp8, optim
+for name in {LIBRARIES}:
+    replaced(name, os.path.join({PACKAGE!r}, name))
+x = torch.randn(64, 512, device="cuda").bfloat16()
+q, k = fp8.quantize(x)
+assert torch.equal(fp8.dequantize(q, k, torch.bfloat16), fp8.roundtrip(x))
+assert torch.equal(q.view(torch.uint8), (x * torch.exp2(-k.float()).bfloat16()).to(q.dtype).view(torch.uint8))
+p = torch.zeros(300, device="cuda")
+p.grad = torch.full((300,), 2.0, device="cuda")
+assert abs(float(optim.clip_grad_norm_([p], 1.0)) - 2.0 * 300**0.5) < 1e-4
+for name in {LIBRARIES}:
+    assert str(os.stat("elysium_wan_amd/" + name).st_ino) in mapped(name), name
+""")
