@@ -1452,15 +1452,17 @@ static unsigned blocks_for_waves(int64_t waves) {
 // (rows_units): a wave per row up to kMaxWaveVpl units, a block per row above,
 // of as many waves as keep at most 4 vectors per lane in each: 4 waves to 16
 // units, 8 to 32, 16 to kMaxRowUnits (32,768 bf16 or 16,384 fp32 columns).
-// Against the split path, which reads x twice and makes three launches:
-// [4096, 6144] fp32 quantizes in 21.2 us against 37.2 (5.9 against 3.4 TB/s),
-// [4096, 20480] bf16 in 43 against 66, [2048, 16384] fp32 in 28 against 50,
-// [2048, 32768] bf16 in 34 against 55, and one row of 32,768 bf16 in 4.2
-// against 10.8 (launch-bound).
+// Against the split path, which reads x twice in two launches (from graphs,
+// buffers in turn): [4096, 6144] fp32 quantizes in 21.8 us against 37.6 (5.8
+// against 3.3 TB/s), [4096, 20480] bf16 in 41.6 against 66.4, [2048, 16384]
+// fp32 in 28.5 against 50.6, [2048, 32768] bf16 in 33.7 against 55.3, 64 rows
+// of 32,768 bf16 in 4.4 against 6.9, and one in 3.3 against 4.9.
 constexpr int kMaxWaveVpl = 6;
 constexpr int kMaxRowUnits = 64;
 // Longer rows than this, and rows that are not whole aligned vectors, are
-// called with the split path's workspace, whether it is used or not.
+// called with the split path's workspace, whether it is used or not: callers
+// size it by ely_fp8_workspace_bytes for every shape, and what was refused
+// without it when these rows took the split path still is.
 constexpr int kNoWorkspaceUnits = 16;
 
 template <int FMT, bool BF16, int VPL>
@@ -1717,6 +1719,7 @@ static void dequantize_impl(const uint8_t* q, const int32_t* k, int64_t rows, in
         return launch_dequant_flat<FMT, BF16OUT, false>(q, k, n, cols, out, s);
     const int64_t segs = (cols + kDeqSegCodes - 1) / kDeqSegCodes;
     if (rows > INT64_MAX / segs) fail(ELY_EINVAL, "too many segments");
+    // past the element-wise kernel's grid these rows stay refused, whichever kernel takes them
     const unsigned any_blocks = blocks_for_waves(rows * segs);
     // Few narrow rows to fp32: the element-wise kernel's wave a row is done
     // sooner than the flat one's (124 rows of 33 codes 2.35 us against 2.96, 512
@@ -1910,8 +1913,9 @@ int ely_fp8_quantize_noalloc(const void* x, int32_t x_dtype, int64_t rows, int64
         check_shape(rows, cols);
         if (rows * cols > 0 && !x) fail(ELY_EINVAL, "ely_fp8_quantize_noalloc: null x");
         if (rows > 0 && !k) fail(ELY_EINVAL, "ely_fp8_quantize_noalloc: null k");
-        // Only the split path (rows that fit no register path) uses scratch;
-        // its row maxima and partials must fit the static array.  Every
+        // Only the split path (rows that fit no register path) uses scratch,
+        // but every shape that wants_workspace is held to what the static
+        // array takes of row maxima and partials.  Every
         // scratch word the split launches read was written by an earlier
         // launch of the same call, so nothing needs clearing between calls.
         const bool split = rows > 0 && cols > 0 && wants_workspace(cols, x_dtype, x, q, nullptr);

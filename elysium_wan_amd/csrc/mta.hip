@@ -584,7 +584,8 @@ struct AdamArgTable {
     ely_adamw_consts c;
     // as the table's chunk map, a byte a chunk, four to a word: one scalar load
     // against up to six dependent ones of a binary search (21 M elements in 38
-    // tensors: the launch 95.0 -> 92.6 us, the step 113.9 -> 113.2)
+    // tensors: the launch 95.0 -> 92.6 us; the whole step, 114-115 us, shows no
+    // difference beyond its noise)
     uint32_t map[kArgChunks / 4];
     int32_t shift;
     int32_t mapped;
@@ -977,10 +978,11 @@ static void clip_scale(const NormLaunch& nl, const float* coef_dev, void* stream
     int64_t blocks = std::min<int64_t>((nl.tiles + kBlock / kWave - 1) / (kBlock / kWave), most);
     // The norm read its tiles first to last; a list the 256 MB MALL holds is
     // scaled last to first, so that it begins on what the L2s hold too, with a
-    // block's tiles on the XCD that summed them (the scale of 88 MB of fp32
-    // 31.8 -> 26.4 us, of 134 MB of bf16 39.9 -> 37.7).  Larger lists measured
-    // the same or worse that way (516 MB of fp32 155 -> 157 us).  It takes
-    // blocks in whole groups of kXcds, which a cap may not leave room for.
+    // block's tiles on the XCD that summed them (norm and scale of 88 MB of fp32
+    // 48.9 -> 47.1 us, of 250 MB 122.6 -> 119.6; bf16, and lists below 60 MB, the
+    // same within 2 %).  Larger lists measured the same or worse that way (516
+    // MB of fp32 155 -> 157 us).  It takes blocks in whole groups of kXcds, which
+    // a cap may not leave room for.
     const int64_t grouped = (blocks + kXcds - 1) / kXcds * kXcds;
     const int32_t last_first = grouped <= most && nl.tiles * nl.tile * (nl.dt == ELY_BF16 ? 2 : 4) <= (int64_t)256 << 20;
     if (last_first) blocks = grouped;

@@ -147,12 +147,17 @@ int64_t ely_fp8_workspace_bytes(int64_t rows, int64_t cols, int32_t x_dtype);
  * and torch's round-to-nearest-even conversion.  Per-tensor scaling is
  * rows = 1.  x: [rows, cols] bf16 or fp32; q: [rows, cols] bytes, or NULL to
  * compute k alone (fp8.scale_exp); k: [rows] int32.
- * A row that fits no register path is read twice (its |x|max, then its
- * codes), except one row of at least 64 MiB given the larger workspace: its exponent is guessed from every
- * 61st 2,048-element segment and the codes are made at the guess in the
- * same pass that finds |x|max (as ely_fp8_quantize_hint does), a second
- * pass following only when the guess was wrong.  The bytes are the same
- * either way. */
+ * A row that fits no register path (of over 32,768 bf16 or 16,384 fp32
+ * columns, or shorter than a vector) is read twice (its |x|max, then its
+ * codes), except one row of at least 64 MiB given the larger workspace: its
+ * exponent is guessed from every 61st 2,048-element segment and the codes are
+ * made at the guess in the same pass that finds |x|max (as
+ * ely_fp8_quantize_hint does), a second pass following only when the guess
+ * was wrong.  The bytes are the same either way.
+ * workspace: ely_fp8_workspace_bytes(rows, cols, x_dtype), asked for
+ * (ELY_EWORKSPACE) by every row of over 8,192 bf16 or 4,096 fp32 columns and
+ * by rows that are no whole 16-byte vectors at aligned addresses, also where
+ * the registers hold them; other rows need none. */
 int ely_fp8_quantize(const void* x, int32_t x_dtype, int64_t rows, int64_t cols, int32_t fmt,
                      uint8_t* q, int32_t* k, void* workspace, int64_t ws_bytes, void* stream);
 
@@ -161,8 +166,10 @@ int ely_fp8_quantize(const void* x, int32_t x_dtype, int64_t rows, int64_t cols,
  * that forbid hipMalloc).  Same results; no workspace argument and no
  * allocation of any kind: the split path (rows longer than the register
  * paths take, e.g. per-tensor scaling) keeps its row maxima in a 1 MiB
- * static device array of the library, one per GPU, so it accepts at most
- * ~131,000 such rows and refuses more with ELY_EINVAL.  Calls that overlap
+ * static device array of the library, one per GPU.  More than ~131,000 rows
+ * are refused with ELY_EINVAL where they are longer than 8,192 bf16 or 4,096
+ * fp32 columns, or no whole 16-byte vectors at aligned addresses, whether
+ * the split path takes them or the registers do.  Calls that overlap
  * on one GPU (different streams, or threads without ordering) share that
  * array and race; calls on one stream are ordered and safe. */
 int ely_fp8_quantize_noalloc(const void* x, int32_t x_dtype, int64_t rows, int64_t cols, int32_t fmt,
