@@ -28,13 +28,14 @@ namespace {
 // A block of W waves moves V 16-byte vectors per lane of a row and ends, a
 // row's pieces across the grid, rows down (a longer list strides).  Launches
 // that touch more than the 256 MB MALL holds stream (nontemporal loads, and
-// the split's stores), one-wave blocks taking the pieces; the others keep to
-// plain accesses, for the rows and the sum are read again soon, in the shapes
-// of fold_shape and split_shape.  Streaming, against a 256-thread block that
+// the split's stores of the sum; its held rows stay in the caches, which took
+// the split of the table below from 147 to 143 us), one-wave blocks taking the
+// pieces; the others keep to plain accesses, for the rows and the sum are read
+// again soon, in the shapes of fold_shape and split_shape.  Streaming, against a 256-thread block that
 // loops over its row, buffers in turn, a third of the rows held: 32,768 x
-// 2,560 fp32 split 166 -> 146 us (5.1 -> 5.8 TB/s) and fold of the held 77 ->
-// 60, bf16 84 -> 76 and 40 -> 40; 32,768 x 1,001 bf16, element by element
-// before, 90 -> 43 and 40 -> 21.
+// 2,560 fp32 split 166 -> 143 us (5.1 -> 5.9 TB/s) and fold of the held 77 ->
+// 58, bf16 84 -> 75 and 40 -> 39; 32,768 x 1,001 bf16, element by element
+// before, 90 -> 44 and 40 -> 21.
 constexpr int64_t kMallBytes = (int64_t)256 << 20;
 constexpr int64_t kRowGrid = 65535;
 
@@ -154,7 +155,7 @@ __device__ __forceinline__ void copy_piece(char* o, const char* x, int64_t d, in
         if (v0 + u * T < nvec) t[u] = ld_row<NT>(x + (v0 + u * T) * 16);
 #pragma unroll
     for (int u = 0; u < V; ++u)
-        if (v0 + u * T < nvec) st_row<NT>(o + (v0 + u * T) * 16, t[u]);
+        if (v0 + u * T < nvec) st_row<false>(o + (v0 + u * T) * 16, t[u]);
     if (piece != (int)gridDim.x - 1) return;
     for (int64_t c = nvec * 16 + threadIdx.x; c < d * ESZ; c += T) o[c] = x[c];
 }
@@ -164,7 +165,7 @@ __device__ __forceinline__ void copy_piece(char* o, const char* x, int64_t d, in
 // acc[r] + (a[r] + 0.0), each add rounded to the dtype; a held row
 // (slot[r] >= 0) is copied to held_out[slot[r]] bit for bit and acc[r] is
 // left for its resolve.
-template <bool BF16, int V, int W, bool NT>
+template <bool BF16, int V, int W, bool NTL, bool NTS>
 __global__ __launch_bounds__(kWave * W) void rows_split_kernel(void* __restrict__ acc, const void* __restrict__ a,
                                                                const int32_t* __restrict__ slot,
                                                                void* __restrict__ held_out, int64_t n_rows,
@@ -174,9 +175,9 @@ __global__ __launch_bounds__(kWave * W) void rows_split_kernel(void* __restrict_
         const int64_t s = slot[r];
         const char* x = static_cast<const char*>(a) + r * row_bytes;
         if (s < 0)
-            fold_piece<BF16, V, W, NT, NT>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, blockIdx.x, first, vec);
+            fold_piece<BF16, V, W, NTL, NTS>(static_cast<char*>(acc) + r * row_bytes, x, nullptr, d, blockIdx.x, first, vec);
         else if (s < n_held)  // the host numbers the held rows 0..n_held-1
-            copy_piece<BF16, V, W, NT>(static_cast<char*>(held_out) + s * row_bytes, x, d, blockIdx.x, vec);
+            copy_piece<BF16, V, W, NTL>(static_cast<char*>(held_out) + s * row_bytes, x, d, blockIdx.x, vec);
     }
 }
 
@@ -192,14 +193,17 @@ dim3 rows_grid(int64_t rows, int64_t nvec, int64_t span, int64_t threads) {
 // 2 and 4 waves of a vector a lane up to 64, 128 and 256 vectors, 4 waves of two
 // up to 512.  (A row of two blocks, the second nearly empty, puts the empty
 // ones on every second XCD: 320 vectors 12.4 us against 9.8 in one-wave
-// pieces.)  Past 512 a row is cut in pieces again.  The fold of few rows, and
+// pieces.)  Past 512 a row is cut in pieces again (640 vectors in three blocks
+// of two waves folded 6.5 us against 8.2 over and over, but 22.2 against 21.3
+// within the launches of a whole table).  The fold of few rows, and
 // of long bf16 rows, is the faster on one-wave pieces; so is the split of more
-// than 32 MB of bf16, two vectors a lane.
+// than 32 MB of bf16 (the sum's stores streamed) or of long fp32 rows, two
+// vectors a lane.
 // The launches of four microbatches (split and fold each), from a graph, in us,
 // with a looping 256-thread block per row / one-wave pieces at every size /
-// these: fp32 256 x 1,024 17.1 / 18.4 / 16.5, 4,096 x 768 41.8 / 46.9 / 41.9,
-// 8,192 x 1,024 82 / 87 / 81, 16,384 x 1,600 230 / 252 / 235; bf16 256 x 768
-// 19.6 / 22.5 / 19.2, 8,192 x 2,048 88 / 95 / 89, 32,768 x 768 179 / 140 / 138.
+// these: fp32 256 x 1,024 17.1 / 18.1 / 16.6, 4,096 x 768 41.8 / 47.0 / 42.5,
+// 8,192 x 1,024 82 / 87 / 81, 16,384 x 1,600 230 / 251 / 235; bf16 256 x 768
+// 19.6 / 22.5 / 18.9, 8,192 x 2,048 88 / 96 / 90, 32,768 x 768 179 / 142 / 139.
 // One by one, a third of 8,192 x 1,024 fp32 rows folded again and again: 5.7 /
 // 7.8 / 5.5; 16,384 x 1,600 split 42.5 / 49.0 / 42.0.
 struct RowShape {
@@ -211,12 +215,11 @@ RowShape fold_shape(int64_t rows, int64_t nvec, bool bf16) {
     if (nvec <= 4 * kWave) return {1, 4};
     if (nvec <= 7 * kWave) return {2, 4};
     if (nvec <= 8 * kWave) return {1, 4};
-    if (nvec <= 12 * kWave) return {2, 2};
     return {1, 1};
 }
 RowShape split_shape(int64_t rows, int64_t nvec, bool bf16) {
     if (nvec <= kWave) return {1, 1};
-    if (bf16 && rows * nvec * 16 > kMallBytes / 8) return {2, 1};
+    if (rows * nvec * 16 > kMallBytes / 8 && (bf16 || nvec > 7 * kWave)) return {2, 1};
     if (nvec <= 2 * kWave) return rows <= 512 ? RowShape{1, 1} : RowShape{1, 2};
     if (nvec <= 4 * kWave || rows <= 512 || (rows <= 1024 && nvec > 8 * kWave)) return {1, 4};
     if (nvec <= 8 * kWave) return {2, 4};
@@ -263,8 +266,7 @@ extern "C" int ely_rows_fold(void* acc, const void* a, const int64_t* a_rows, co
             constexpr bool B = decltype(bf16)::value;
             if (3 * n_idx * d * esz > kMallBytes) return launch(rows_fold_kernel<B, 1, 1, true>, 1, 1);
             const RowShape sh = vec ? fold_shape(n_idx, nvec, B) : RowShape{1, 4};
-            if (sh.v == 2 && sh.w == 4) launch(rows_fold_kernel<B, 2, 4, false>, 2, 4);
-            else if (sh.v == 2) launch(rows_fold_kernel<B, 2, 2, false>, 2, 2);
+            if (sh.v == 2) launch(rows_fold_kernel<B, 2, 4, false>, 2, 4);
             else if (sh.w == 4) launch(rows_fold_kernel<B, 1, 4, false>, 1, 4);
             else if (sh.w == 2) launch(rows_fold_kernel<B, 1, 2, false>, 1, 2);
             else launch(rows_fold_kernel<B, 1, 1, false>, 1, 1);
@@ -292,13 +294,14 @@ extern "C" int ely_rows_split(void* acc, const void* a, const int32_t* slot, voi
         };
         const auto shape = [&](auto bf16) {
             constexpr bool B = decltype(bf16)::value;
-            if (2 * n_rows * d * esz > kMallBytes) return launch(rows_split_kernel<B, 2, 1, true>, 2, 1);
+            if (2 * n_rows * d * esz > kMallBytes) return launch(rows_split_kernel<B, 2, 1, true, true>, 2, 1);
             const RowShape sh = vec ? split_shape(n_rows, nvec, B) : RowShape{1, 4};
-            if (sh.v == 2 && sh.w == 4) launch(rows_split_kernel<B, 2, 4, false>, 2, 4);
-            else if (sh.v == 2) launch(rows_split_kernel<B, 2, 1, false>, 2, 1);
-            else if (sh.w == 4) launch(rows_split_kernel<B, 1, 4, false>, 1, 4);
-            else if (sh.w == 2) launch(rows_split_kernel<B, 1, 2, false>, 1, 2);
-            else launch(rows_split_kernel<B, 1, 1, false>, 1, 1);
+            if (sh.v == 2 && sh.w == 4) launch(rows_split_kernel<B, 2, 4, false, false>, 2, 4);
+            else if (sh.v == 2 && B && n_rows * d * esz > kMallBytes / 8) launch(rows_split_kernel<B, 2, 1, false, true>, 2, 1);
+            else if (sh.v == 2) launch(rows_split_kernel<B, 2, 1, false, false>, 2, 1);
+            else if (sh.w == 4) launch(rows_split_kernel<B, 1, 4, false, false>, 1, 4);
+            else if (sh.w == 2) launch(rows_split_kernel<B, 1, 2, false, false>, 1, 2);
+            else launch(rows_split_kernel<B, 1, 1, false, false>, 1, 1);
         };
         dtype == ELY_BF16 ? shape(std::true_type()) : shape(std::false_type());
         check_launch("rows_split_kernel");

@@ -243,24 +243,35 @@ def test_tied_fold_at_any_width_equals_the_dense_fold(dtype, d):
 @pytest.mark.parametrize("n", [300, 700, 1100])
 @pytest.mark.parametrize("vecs", [1, 63, 64, 65, 128, 129, 256, 257, 448, 449, 512, 513, 768, 769])
 def test_tied_fold_in_every_block_shape_equals_the_dense_fold(dtype, n, vecs):
-    from elysium_wan_amd.accumulate import TiedRowFold
-
     epv = 8 if dtype == torch.bfloat16 else 4
     for d in (vecs * epv, vecs * epv + 3):
-        g = torch.Generator(device="cuda").manual_seed(vecs)
-        t = n - 90
-        hs = [torch.randn(n, d, generator=g, device="cuda").to(dtype) for _ in range(2)]
-        ids = [torch.randperm(n, generator=g, device="cuda")[:t].sort().values for _ in range(2)]
-        es = [torch.randn(t, d, generator=g, device="cuda").to(dtype) for _ in range(2)]
-        say("tied fold shapes", dtype, n, d)
-        fold = TiedRowFold(n, range(2))
-        for k in range(2):
-            fold.add_head(k, hs[k], ids[k])
-        for k in range(2):
-            fold.add_embed(k, es[k])
-        parts = []
-        for k in range(2):
-            e = torch.zeros(n, d, dtype=dtype, device="cuda")
-            e[ids[k]] = es[k]
-            parts.append(hs[k] + e)
-        assert torch.equal(fold.result(), parts[0] + parts[1])
+        _tied_fold_equals_the_dense_fold(dtype, n, d)
+
+
+# past 32 MB, and past the size from which launches stream
+@pytest.mark.parametrize("dtype,n,d", [(torch.bfloat16, 9000, 2048), (torch.bfloat16, 17000, 1001), (torch.float32, 9000, 2050), (torch.float32, 9000, 1025),
+                                       (torch.float32, 16500, 2051), (torch.bfloat16, 33000, 2053)])
+def test_tied_fold_of_large_tables_equals_the_dense_fold(dtype, n, d):
+    _tied_fold_equals_the_dense_fold(dtype, n, d)
+
+
+def _tied_fold_equals_the_dense_fold(dtype, n, d):
+    from elysium_wan_amd.accumulate import TiedRowFold
+
+    g = torch.Generator(device="cuda").manual_seed(d)
+    t = n - 90
+    hs = [torch.randn(n, d, generator=g, device="cuda").to(dtype) for _ in range(2)]
+    ids = [torch.randperm(n, generator=g, device="cuda")[:t].sort().values for _ in range(2)]
+    es = [torch.randn(t, d, generator=g, device="cuda").to(dtype) for _ in range(2)]
+    say("tied fold shapes", dtype, n, d)
+    fold = TiedRowFold(n, range(2))
+    for k in range(2):
+        fold.add_head(k, hs[k], ids[k])
+    for k in range(2):
+        fold.add_embed(k, es[k])
+    parts = []
+    for k in range(2):
+        e = torch.zeros(n, d, dtype=dtype, device="cuda")
+        e[ids[k]] = es[k]
+        parts.append(hs[k] + e)
+    assert torch.equal(fold.result(), parts[0] + parts[1])
